@@ -415,6 +415,13 @@ __device__ __forceinline__ Q8Lane quantize32(float x) {
     return q;
 }
 
+// A Q8 code of element e as the fp16 bits the operand plane holds (half_slot):
+// the code itself, or code / 16 for the elements of high nibbles.
+__device__ __forceinline__ uint32_t half_operand(int code, int e) {
+    const float v = static_cast<float>(code);
+    return f2h(e < 16 ? v : v * 0.0625f);
+}
+
 // One Q8_1 block from P lanes (P = 2 or 4): lane l holds elements
 // (32/P) * part .. +32/P-1 of its block, part = l / (64/P); the partners are
 // lanes l ^ 32 (and l ^ 16 for P = 4).  Same bits as quantize32: max is

@@ -1,0 +1,12 @@
+// The 64-block form of the fp16-operand gate / up kernel (moe_half.hpp), built
+// with the iterative ILP machine scheduler (Makefile).
+#include "moe_half.hpp"
+
+namespace moe {
+
+hipError_t launch_gate_up_half_full(const FfnArgs &a, unsigned grid, hipStream_t s) {
+    k_gate_up_half<true, false><<<grid, kHtThreads, 0, s>>>(a);
+    return hipGetLastError();
+}
+
+}  // namespace moe

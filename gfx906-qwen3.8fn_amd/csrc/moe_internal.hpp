@@ -95,7 +95,26 @@ struct RouteOut {
 struct Act {               // split-plane Q8 rows
     uint8_t *codes;        // [rows][blocks][32]
     uint32_t *heads;       // [rows][blocks]
+    uint16_t *half = nullptr;   // [rows][blocks][32] fp16 MFMA operands (half_slot), or null: not written
 };
+
+// The fp16 operand plane of an MFMA projection.  v_mfma_f32_32x32x16_f16
+// takes one fragment (16 elements) of a block per issue: lane half h supplies
+// the 8 elements of nibble dword 2f + h of the weight chunk (bytes 8f + 4h ..
+// + 3).  A nibble n left in place under a mask, read as an fp16 bit pattern,
+// is the subnormal n * 2^-24 at bits 0..3 and n * 2^-20 at bits 4..7, so the
+// weights need no conversion; the activation of a high nibble (elements
+// 16..31) is stored as code / 16 to make up for its position.  Every product
+// is then n * code * 2^-24 and every partial sum an integer (below 2^15) times
+// 2^-24: the MFMA's fp32 result is exactly float(I_f) * 2^-24.
+// The kernels that read it take rows of at most kHalfMaxBlocks blocks.
+inline constexpr int kHalfMaxBlocks = 64;
+// Element e of a block sits at half_slot(e): [lane half][fragment][high
+// nibble][byte odd][byte pair].
+__host__ __device__ constexpr int half_slot(int e) {
+    const int byte = e & 15, hi = e >> 4, f = byte >> 3, h = (byte >> 2) & 1, j = byte & 3;
+    return ((2 * h + f) * 2 + hi) * 4 + 2 * (j & 1) + (j >> 1);
+}
 
 // ----------------------------------------------------------------------------
 // Kernel launchers (moe_kernels.hip).  All return hipGetLastError() after the
@@ -179,14 +198,17 @@ hipError_t launch_down(const FfnArgs &a, bool mfma, hipStream_t s);
 // Int8-MFMA kernels over the MFMA items (moe_mfma.hip).
 hipError_t launch_gate_up_mfma(const FfnArgs &a, hipStream_t s);
 hipError_t launch_down_mfma(const FfnArgs &a, hipStream_t s);
+// Rows of at most 64 blocks, on fp16 operands (moe_half.hip, moe_half_full.hip).
+hipError_t launch_gate_up_half(const FfnArgs &a, hipStream_t s);
+hipError_t launch_gate_up_half_full(const FfnArgs &a, unsigned grid, hipStream_t s);
 
 // One Q4_0 matrix (planes, rows padded to a multiple of 32) against N
-// columns in split Q8 planes, in the reference MMVQ fp32 order, on int8 MFMA
-// (moe_mfma.hip); used by moe_linear for wide column counts.
+// Q8_1 columns, in the reference MMVQ fp32 order, on MFMA (moe_mfma.hip);
+// used by moe_linear for wide column counts.
 struct LinearMfmaArgs {
     const uint8_t *codes;     // [Mp][nb][16 B]
     const uint16_t *scales;   // [Mp/8][nb][8]
-    Act xq;                   // [N][nb] planes, read when q8 is null
+    Act xq;                   // [N][nb] operand and head planes (xq.half, xq.heads), read when q8 is null
     const uint8_t *q8;        // canonical Q8_1 columns [N][nb][36 B] {d, s, qs[32]}, or null
     float *y;                 // [N][M]
     int nb, M, N;

@@ -19,33 +19,109 @@ namespace moe {
 namespace {
 
 // ------------------------------------------------------------ quantizers ---
-// One thread per element; 32-lane groups are whole Q8 blocks.
+// 64 blocks per 256-thread workgroup: wave w takes blocks 16w .. 16w + 15 of
+// the workgroup's, lane l elements 8 (l / 16) .. + 7 of block l % 16 (two
+// 16-byte loads), reduced by quantize_part<4> (aligned subtrees of the
+// reference's butterfly, the same bytes as quantize32).  `elements` is a
+// multiple of 32, so the bound check keeps or drops whole blocks; every lane
+// takes part in the shuffles.  store(block, part, q) gets each lane's part.
+template<class Store>
+__device__ __forceinline__ void quantize_group(const float *__restrict__ x, size_t blk0, size_t elements, Store &&store) {
+    const int lane = static_cast<int>(threadIdx.x & 63), wave = static_cast<int>(threadIdx.x >> 6);
+    const int part = lane >> 4;
+    const size_t block = blk0 + 16 * wave + (lane & 15);
+    // The workgroup's 8 KB through one buffer descriptor (x needs only
+    // 4-byte alignment; past `elements` the loads read zeros).
+    const size_t left = elements - blk0 * 32;
+    const auto xr = buffer_rsrc(x + blk0 * 32, static_cast<uint32_t>(std::min<size_t>(left, 2048) * 4));
+    const uint32_t off = static_cast<uint32_t>((16 * wave + (lane & 15)) * 128 + 32 * part);
+    const uint4 a = buffer_load16(xr, off, 0), b = buffer_load16(xr, off, 16);
+    float v[8] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z), __uint_as_float(a.w),
+                  __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w)};
+    const Q8Part<4> q = quantize_part<4>(v);
+    if (block * 32 < elements) store(block, part, q);
+}
+
+// Elements 8 part .. + 7 of a block into its fp16 operand slots: fragment
+// part & 1, low nibbles (part < 2) or high; for lane half h the four elements
+// are one 8-byte store.
+__device__ __forceinline__ void store_half_part(uint16_t *half, size_t block, int part, const uint32_t (&codes)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        uint32_t v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            v[j] = half_operand(static_cast<int8_t>(codes[h] >> (8 * j)), part < 2 ? 0 : 16);
+        *reinterpret_cast<uint2 *>(half + block * 32 + half_slot(8 * part + 4 * h)) =
+            make_uint2(v[0] | v[2] << 16, v[1] | v[3] << 16);
+    }
+}
+
+// The planes that are there: codes, the fp16 operands, heads.
+__device__ __forceinline__ void store_planes(const Act &out, size_t block, int part, const Q8Part<4> &q, int *error) {
+    if (out.codes) *reinterpret_cast<uint2 *>(out.codes + block * 32 + 8 * part) = make_uint2(q.codes[0], q.codes[1]);
+    if (out.half) store_half_part(out.half, block, part, q.codes);
+    if (part == 0) {
+        out.heads[block] = q.head;
+        if (q.flags) atomicOr(error, q.flags);
+    }
+}
+
+// One element per lane, a block per 32 lanes: short batches, whose time is
+// one wave's latency.
 template<bool Canonical>
-__global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ x, uint8_t *codes,
-                                                  uint32_t *heads, size_t elements, int *error) {
+__global__ __launch_bounds__(256) void k_quantize_short(const float *__restrict__ x, Act out, size_t elements, int *error) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= elements) return;   // elements is a multiple of 32: whole groups exit together
     const Q8Lane q = quantize32(x[i]);
     const size_t block = i >> 5;
     const int lane = static_cast<int>(i & 31);
     if constexpr (Canonical) {
-        codes[block * 36 + 4 + lane] = static_cast<uint8_t>(q.code);
-        if (lane == 0) *reinterpret_cast<uint32_t *>(codes + block * 36) = q.head;
+        out.codes[block * 36 + 4 + lane] = static_cast<uint8_t>(q.code);
+        if (lane == 0) *reinterpret_cast<uint32_t *>(out.codes + block * 36) = q.head;
     } else {
-        codes[block * 32 + lane] = static_cast<uint8_t>(q.code);
-        if (lane == 0) heads[block] = q.head;
+        if (out.codes) out.codes[block * 32 + lane] = static_cast<uint8_t>(q.code);
+        if (out.half) out.half[block * 32 + half_slot(lane)] = static_cast<uint16_t>(half_operand(q.code, lane));
+        if (lane == 0) out.heads[block] = q.head;
     }
     if (lane == 0 && q.flags) atomicOr(error, q.flags);
 }
 
-__global__ __launch_bounds__(256) void k_canonical_to_planes(const uint8_t *q8, uint8_t *codes,
-                                                             uint32_t *heads, size_t blocks) {
+// fp32 rows -> canonical 36-byte blocks (out.codes, 4-byte aligned) or planes,
+// eight elements a lane (bound by VALU: the IEEE divisions and the lane
+// butterflies, here a quarter as many a value).  Canonical, width 2048, us, one
+// element a lane -> eight: 1,032 columns 7.7 -> 4.2, 4,096 25.0 -> 9.9.
+template<bool Canonical>
+__global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ x, Act out, size_t elements, int *error) {
+    quantize_group(x, static_cast<size_t>(blockIdx.x) * 64, elements, [&](size_t block, int part, const Q8Part<4> &q) {
+        if constexpr (Canonical) {
+            uint32_t *dst = reinterpret_cast<uint32_t *>(out.codes + block * 36);
+            dst[1 + 2 * part] = q.codes[0];
+            dst[2 + 2 * part] = q.codes[1];
+            if (part == 0) {
+                dst[0] = q.head;
+                if (q.flags) atomicOr(error, q.flags);
+            }
+        } else {
+            store_planes(out, block, part, q, error);
+        }
+    });
+}
+
+__global__ __launch_bounds__(256) void k_canonical_to_planes(const uint8_t *q8, Act out, size_t blocks) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= blocks * 9) return;
     const size_t b = i / 9, w = i % 9;
     const uint32_t v = reinterpret_cast<const uint32_t *>(q8)[i];
-    if (w == 0) heads[b] = v;
-    else reinterpret_cast<uint32_t *>(codes)[b * 8 + (w - 1)] = v;
+    if (w == 0) { out.heads[b] = v; return; }
+    reinterpret_cast<uint32_t *>(out.codes)[b * 8 + (w - 1)] = v;
+    if (out.half) {   // elements 4 (w - 1) .. + 3: one lane half's low or high nibbles of a fragment
+        const int e = static_cast<int>(4 * (w - 1));
+        uint32_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = half_operand(static_cast<int8_t>(v >> (8 * j)), e);
+        *reinterpret_cast<uint2 *>(out.half + b * 32 + half_slot(e)) = make_uint2(o[0] | o[2] << 16, o[1] | o[3] << 16);
+    }
 }
 
 __global__ __launch_bounds__(256) void k_planes_to_canonical(const uint8_t *codes, const uint32_t *heads,
@@ -287,6 +363,7 @@ __global__ __launch_bounds__(1024) void k_prepare_small(GroupParams p, const flo
         const size_t block = i >> 5;
         const int lane = static_cast<int>(i & 31);
         xq.codes[block * 32 + lane] = static_cast<uint8_t>(q.code);
+        if (xq.half) xq.half[block * 32 + half_slot(lane)] = static_cast<uint16_t>(half_operand(q.code, lane));
         if (lane == 0) {
             xq.heads[block] = q.head;
             if (q.flags) atomicOr(p.error, q.flags);
@@ -413,8 +490,6 @@ __device__ int weight_flags(const GroupParams &p, int t0) {
     return flags;
 }
 
-constexpr int kQuantPer = 8;   // quantized elements per thread in k_mark_quantize
-
 // Step 1: blocks [0, mark_blocks) set bitmap bits (one thread per token),
 // the rest quantize x.  The bitmap is [W][Ep] (word-major) so the
 // per-expert prefix kernel reads it coalesced.
@@ -436,34 +511,8 @@ __global__ __launch_bounds__(256) void k_mark_quantize(GroupParams p, int mark_b
         if (flags) atomicOr(p.error, flags);
         return;
     }
-    // A workgroup quantizes 64 blocks (2048 consecutive floats): wave w takes
-    // blocks 16w .. 16w + 15, lane l elements 8 (l / 16) .. + 7 of block
-    // 16w + l % 16 (two 16-byte loads, one 8-byte code store), reduced by
-    // quantize_part<4> (aligned subtrees of the reference's butterfly, the same
-    // bytes as quantize32).  q_elements is a multiple of 32, so the bound check
-    // keeps or drops whole blocks; every lane takes part in the shuffles.
-    static_assert(kQuantPer == 8, "k_mark_quantize: 8 elements per lane");
-    const int lane = static_cast<int>(threadIdx.x & 63), wave = static_cast<int>(threadIdx.x >> 6);
-    const int part = lane >> 4;
-    const size_t blk0 = static_cast<size_t>(blockIdx.x - mark_blocks) * 64;
-    const size_t block = blk0 + 16 * wave + (lane & 15);
-    const bool in = block * 32 < q_elements;
-    // The workgroup's 8 KB through one buffer descriptor (x needs only
-    // 4-byte alignment; past q_elements the loads read zeros).
-    const size_t left = q_elements - blk0 * 32;
-    const auto xr = buffer_rsrc(x + blk0 * 32, static_cast<uint32_t>(std::min<size_t>(left, 2048) * 4));
-    const uint32_t off = static_cast<uint32_t>((16 * wave + (lane & 15)) * 128 + 32 * part);
-    const uint4 a = buffer_load16(xr, off, 0), b = buffer_load16(xr, off, 16);
-    float v[kQuantPer] = {__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z), __uint_as_float(a.w),
-                          __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), __uint_as_float(b.w)};
-    const Q8Part<4> q = quantize_part<4>(v);
-    if (in) {
-        *reinterpret_cast<uint2 *>(xq.codes + block * 32 + 8 * part) = make_uint2(q.codes[0], q.codes[1]);
-        if (part == 0) {
-            xq.heads[block] = q.head;
-            if (q.flags) atomicOr(p.error, q.flags);
-        }
-    }
+    quantize_group(x, static_cast<size_t>(blockIdx.x - mark_blocks) * 64, q_elements,
+                   [&](size_t block, int part, const Q8Part<4> &q) { store_planes(xq, block, part, q, p.error); });
 }
 
 // Step 2: one wave per routed expert: exclusive popcount prefix over words.
@@ -1918,24 +1967,38 @@ inline unsigned blocks_for(size_t n, unsigned per) { return static_cast<unsigned
 }  // namespace
 
 // -------------------------------------------------------------- launchers ---
+namespace {
+// Eight elements a lane from the size where that still gives every CU a
+// workgroup (2,048 elements each).  us, one element a lane / eight, width 2048:
+// 1 column 1.90 / 2.23, 64 2.08 / 2.50, 128 2.44 / 2.51, 256 3.14 / 2.57, 512
+// 4.65 / 3.11.
+constexpr size_t kQuantizeShort = size_t{256} * 2048;
+
+template<bool Canonical>
+void launch_quantize(const float *x, Act out, size_t n, int *error, hipStream_t s) {
+    if (n < kQuantizeShort) k_quantize_short<Canonical><<<blocks_for(n, 256), 256, 0, s>>>(x, out, n, error);
+    else k_quantize<Canonical><<<blocks_for(n, 2048), 256, 0, s>>>(x, out, n, error);
+}
+}  // namespace
+
 hipError_t launch_quantize_canonical(const float *x, void *q8, int width, int columns, int *error,
                                      hipStream_t s) {
     const size_t n = static_cast<size_t>(width) * columns;
-    k_quantize<true><<<blocks_for(n, 256), 256, 0, s>>>(x, static_cast<uint8_t *>(q8), nullptr, n, error);
+    launch_quantize<true>(x, Act{static_cast<uint8_t *>(q8), nullptr}, n, error, s);
     return hipGetLastError();
 }
 
 hipError_t launch_quantize_planes(const float *x, Act out, int width, int columns, int *error,
                                   hipStream_t s) {
     const size_t n = static_cast<size_t>(width) * columns;
-    k_quantize<false><<<blocks_for(n, 256), 256, 0, s>>>(x, out.codes, out.heads, n, error);
+    launch_quantize<false>(x, out, n, error, s);
     return hipGetLastError();
 }
 
 hipError_t launch_canonical_to_planes(const void *q8, Act out, int blocks, hipStream_t s) {
     const size_t n = static_cast<size_t>(blocks) * 9;
-    k_canonical_to_planes<<<blocks_for(n, 256), 256, 0, s>>>(static_cast<const uint8_t *>(q8), out.codes,
-                                                              out.heads, static_cast<size_t>(blocks));
+    k_canonical_to_planes<<<blocks_for(n, 256), 256, 0, s>>>(static_cast<const uint8_t *>(q8), out,
+                                                              static_cast<size_t>(blocks));
     return hipGetLastError();
 }
 
@@ -2007,7 +2070,7 @@ hipError_t launch_prepare(const float *x, const int32_t *ids, const float *weigh
     if (e != hipSuccess) return e;
     const int mark_blocks = static_cast<int>(blocks_for(static_cast<size_t>(tokens), 256));
     const size_t id_lds = static_cast<size_t>(256) * shape.k * 4;
-    k_mark_quantize<<<mark_blocks + blocks_for(q_elements, 256 * kQuantPer), 256, id_lds, s>>>(p, mark_blocks, x, xq,
+    k_mark_quantize<<<mark_blocks + blocks_for(q_elements, 2048), 256, id_lds, s>>>(p, mark_blocks, x, xq,
                                                                                            q_elements);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     k_word_prefix<<<blocks_for(static_cast<size_t>(shape.E), 4), 256, 0, s>>>(p);

@@ -128,7 +128,7 @@ size_t bank_layout(const Shape &s, bool down_q41, size_t off[7]) {
 }
 
 struct WsLayout {
-    size_t xq_codes, xq_heads, mq_codes, mq_heads, pair_token, pair_rank, pos_of, counts, offsets,
+    size_t xq_codes, xq_half, xq_heads, mq_codes, mq_heads, pair_token, pair_rank, pos_of, counts, offsets,
         stream_items, mfma_items, item_counts, bitmap, wprefix, contrib, diag_error, total;
 };
 
@@ -141,6 +141,7 @@ WsLayout ws_layout(const Shape &s, int N) {
     size_t p = 0;
     auto take = [&](size_t bytes) { const size_t at = p; p = round_up(p + bytes, 256); return at; };
     w.xq_codes = take(static_cast<size_t>(N) * nbh * 32);
+    w.xq_half = take(nbh <= moe::kHalfMaxBlocks ? static_cast<size_t>(N) * nbh * 64 : 0);
     w.xq_heads = take(static_cast<size_t>(N) * nbh * 4);
     w.mq_codes = take(P * nbi * 32);
     w.mq_heads = take(P * nbi * 4);
@@ -166,7 +167,8 @@ int finish_create(moe_ffn_layer *L) {
     if (hipMalloc(&L->ws_mem, w.total) != hipSuccess) return hipErrorOutOfMemory;
     L->ws_bytes = w.total;
     auto *b = static_cast<uint8_t *>(L->ws_mem);
-    L->xq = Act{b + w.xq_codes, reinterpret_cast<uint32_t *>(b + w.xq_heads)};
+    L->xq = Act{b + w.xq_codes, reinterpret_cast<uint32_t *>(b + w.xq_heads),
+                reinterpret_cast<uint16_t *>(b + w.xq_half)};
     L->mq = Act{b + w.mq_codes, reinterpret_cast<uint32_t *>(b + w.mq_heads)};
     L->routes.pair_token = reinterpret_cast<int32_t *>(b + w.pair_token);
     L->routes.pair_rank = reinterpret_cast<int32_t *>(b + w.pair_rank);
@@ -382,6 +384,14 @@ moe::FfnArgs base_args(moe_ffn_layer *L, int tokens, int *error) {
     return a;
 }
 
+// The activation planes a batch fills: the fp16 operand plane only when some
+// of its groups can go to an MFMA kernel that reads it.
+Act activation_planes(const moe_ffn_layer *L, bool mfma) {
+    Act xq = L->xq;
+    if (!mfma || L->shape.H / 32 > moe::kHalfMaxBlocks) xq.half = nullptr;
+    return xq;
+}
+
 }  // namespace
 
 extern "C" {
@@ -497,15 +507,16 @@ int run_stage(moe_ffn_layer *L, int stage, const float *x, const int32_t *ids, c
         if (stage == MOE_STAGE_DOWN) return moe::launch_decode_down_fold(d, s);
         return stage >= MOE_STAGE_PREPARE && stage <= MOE_STAGE_FOLD ? hipSuccess : kInvalid;
     }
+    const Act xq = activation_planes(L, L->active_mfma_min > 0);
     switch (stage) {
     case MOE_STAGE_PREPARE:
         if (L->x_q8_in) {   // grouping only, then the given Q8 rows into the activation planes
-            if ((r = moe::launch_prepare(nullptr, ids, weights, tokens, sh, L->xq, L->routes, L->active_mfma_min, error, s)) !=
+            if ((r = moe::launch_prepare(nullptr, ids, weights, tokens, sh, xq, L->routes, L->active_mfma_min, error, s)) !=
                 hipSuccess)
                 return r;
-            return moe::launch_canonical_to_planes(L->x_q8_in, L->xq, tokens * (sh.H / 32), s);
+            return moe::launch_canonical_to_planes(L->x_q8_in, xq, tokens * (sh.H / 32), s);
         }
-        return moe::launch_prepare(x, ids, weights, tokens, sh, L->xq, L->routes, L->active_mfma_min, error, s);
+        return moe::launch_prepare(x, ids, weights, tokens, sh, xq, L->routes, L->active_mfma_min, error, s);
     // With mfma_min == 1 every nonempty group is an MFMA item and the
     // streaming launch would only start empty workgroups.
     case MOE_STAGE_GATE_UP:
@@ -671,7 +682,7 @@ int moe_ffn_expert_gate_up(moe_ffn_layer *L, int expert, const void *x_q8, int c
     const bool mfma = path != MOE_PATH_STREAM;
     const auto s = static_cast<hipStream_t>(stream);
     const Shape &sh = L->shape;
-    hipError_t r = moe::launch_canonical_to_planes(x_q8, L->xq, columns * (sh.H / 32), s);
+    hipError_t r = moe::launch_canonical_to_planes(x_q8, activation_planes(L, mfma), columns * (sh.H / 32), s);
     if (r != hipSuccess) return r;
     if ((r = moe::launch_single_expert_items(sh, L->routes, expert, columns, mfma, s)) != hipSuccess) return r;
     moe::FfnArgs a = base_args(L, columns, error);
@@ -730,7 +741,7 @@ int moe_ffn_expert_run(moe_ffn_layer *L, int expert, const float *x, int columns
     // One forward: quantize x, gate/up + SiLU*up + Q8, down (the work list
     // of the single group is built once, before the warm-up).
     auto pass = [&]() -> hipError_t {
-        hipError_t r = moe::launch_quantize_planes(xd, L->xq, sh.H, columns, err, s);
+        hipError_t r = moe::launch_quantize_planes(xd, activation_planes(L, mfma), sh.H, columns, err, s);
         moe::FfnArgs a = base_args(L, columns, err);
         a.pairs_bound = columns;
         a.mfma_min = mfma ? 1 : 0;

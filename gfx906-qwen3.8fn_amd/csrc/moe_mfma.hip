@@ -23,9 +23,8 @@
 //
 // Work unit = (MFMA item of <= 128 grouped pairs of one expert, row slice),
 // ordered item-major and dealt to the XCDs in chunks (see mfma_unit).
-#include "moe_device.hpp"
+#include "moe_mfma_device.hpp"
 
-#include <algorithm>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -33,83 +32,9 @@
 namespace moe {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-
-constexpr int kSub = 32;                   // tokens per MFMA tile (N)
-constexpr int kSubs = kMfmaTile / kSub;    // tiles per item
 constexpr int kMagic = 0x4B400000;         // bits of 12582912.0f
 constexpr float kMagicF = 12582912.0f;
 constexpr uint32_t kNibbles = 0x0f0f0f0fu;
-
-struct Unit {
-    int item, slice;
-    bool ok;
-};
-
-// blockIdx -> (item, slice).  Workgroup i runs on XCD i % 8; XCD x takes
-// chunks of kUnitChunk consecutive units round-robin (chunk c goes to XCD
-// c % 8), so the units of one item slice share an XCD while the work of the
-// popular experts is spread over all XCDs.
-constexpr int kUnitChunk = 4;
-
-// The dealing permutes each round of 8 * kUnitChunk consecutive ids.  Within
-// an XCD the dispatcher hands consecutive workgroups to its four shader
-// engines in turn (measured: a workgroup's engine follows its position
-// modulo 4 in the XCD's sequence for three quarters of them), so the unit
-// at position p of chunk k is unit (p + k) % 4 of that chunk: the gate/up
-// kernel's token tile `sub` (empty for the tail tiles of small items) then
-// visits every engine instead of pinning the working tiles to one.
-__device__ __forceinline__ int dealt_unit(int id) {
-    const int n = id >> 3, x = id & 7, k = n / kUnitChunk;
-    return (k * 8 + x) * kUnitChunk + (n + k) % kUnitChunk;
-}
-
-// Chunks of kGuChunkRows row slices per XCD (the gate/up kernel): the
-// item-major sequence of (item, row slice) pairs is cut into chunks of
-// kGuChunkRows, chunk c runs on XCD c % 8, and the activations of an item's
-// token tiles, read by every row slice, are fetched into fewer L2s.  Within a
-// chunk, row slice r's token tiles are rotated by r + c over the four
-// positions so each engine sees every tile index.  Chunk rows, layer ms
-// (2048/512, two runs each): 1 (one row slice): 4K 1.47-1.49, 16K 4.61,
-// stack 26.65; 4: 1.47-1.48, 4.53-4.55, 26.56; 8: 1.46-1.47, 4.51-4.56,
-// 26.90; 16 (whole items): 1.48-1.50, 4.52, 27.7 (items dealt whole leave
-// the XCDs unevenly loaded on the stack's 1,032-token layers).
-constexpr int kGuChunkRows = 4;
-constexpr int kGuChunk = kGuChunkRows * kSubs;
-
-__device__ __forceinline__ Unit row_chunk_unit(int count, int slices) {
-    const int id = static_cast<int>(blockIdx.x);
-    const int n = id >> 3, x = id & 7, k = n / kGuChunk, p = n - k * kGuChunk;
-    const int rl = p / kSubs;
-    const int u = (k * 8 + x) * kGuChunk + rl * kSubs + (p + rl + k) % kSubs;
-    Unit r;
-    r.ok = u < count * slices;
-    r.item = r.ok ? u / slices : 0;
-    r.slice = r.ok ? u % slices : 0;
-    return r;
-}
-
-__device__ __forceinline__ Unit mfma_unit(int count, int slices) {
-    const int units = count * slices;
-    const int u = dealt_unit(static_cast<int>(blockIdx.x));
-    Unit r;
-    r.ok = u < units;
-    r.item = r.ok ? u / slices : 0;
-    r.slice = r.ok ? u % slices : 0;
-    return r;
-}
-
-__device__ __forceinline__ float half_lo(uint32_t w) { return h2f(w); }
-__device__ __forceinline__ float half_hi(uint32_t w) { return h2f(w >> 16); }
-
-// 8 fp16 values as an MFMA operand.
-__device__ __forceinline__ v8h pack8(const uint32_t (&w)[4]) {
-    v4i v = {static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
-    return __builtin_bit_cast(v8h, v);
-}
 
 // The fp16 hi halves (s of a Q8_1 head) of 8 heads, zero for blocks >= nb.
 __device__ __forceinline__ v8h head_sums(uint4 h0, uint4 h1, int kb0, int nb) {
@@ -122,22 +47,6 @@ __device__ __forceinline__ v8h head_sums(uint4 h0, uint4 h1, int kb0, int nb) {
         w[e] = lo | hi;
     }
     return pack8(w);
-}
-
-// fp16 -> fp32 conversions the compiler cannot fold into v_fma_mix_f32.  On
-// gfx950 v_fma_mix_f32 issues at about the rate of a conversion (measured:
-// 0.5 wave-instructions per SIMD per ns against 0.9 for v_fma_f32, v_mul_f32
-// and v_add_f32), so a scale used by several products is converted once and
-// the products are plain fp32 fmas.  (Same values: fp16 -> fp32 is exact.)
-__device__ __forceinline__ float cvt_half_lo(uint32_t w) {
-    float r;
-    asm("v_cvt_f32_f16 %0, %1" : "=v"(r) : "v"(w));
-    return r;
-}
-__device__ __forceinline__ float cvt_half_hi(uint32_t w) {
-    float r;
-    asm("v_cvt_f32_f16_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1" : "=v"(r) : "v"(w));
-    return r;
 }
 
 // As scale_block below, with the 16 row scales already in fp32.
@@ -332,19 +241,6 @@ __device__ __forceinline__ void tile_dispatch(const TileArgs &t, int nsub, float
 // middle.  Fragment dots come from two MFMAs per block whose A operands keep
 // only that fragment's bytes (the other half zero); both MFMAs start from 0.
 
-// acc[v] = fma(d4[v], fma(float(I[v]), d8, c4), acc[v]); d4 read as fp16 by
-// v_fma_mix_f32 (lo / hi half of each word).
-__device__ __forceinline__ float fma_mix_lo(uint32_t h2, float t, float acc) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(t), "v"(acc));
-    return r;
-}
-__device__ __forceinline__ float fma_mix_hi(uint32_t h2, float t, float acc) {
-    float r;
-    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h2), "v"(t), "v"(acc));
-    return r;
-}
-
 __device__ __forceinline__ void fragment_scale(float (&acc)[16], v16i I, float d8, float c4, const uint32_t (&d4)[8]) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
@@ -405,7 +301,6 @@ __device__ __forceinline__ void store_dots(const GuTile &t, int b, v16i I0, v16i
 
 // ---- H <= 2048 (one block per reference lane): staged scales and heads,
 // weights and activations prefetched one leaf pair ahead.
-constexpr int kGuMaxBlocks = 64;
 
 struct GuStage {
     const uint32_t *d4;   // LDS [nb][32 halfs] of this wave's rows (row 16h + v at half 16h + v)
@@ -488,57 +383,6 @@ __device__ __forceinline__ void leaf_staged(const GuTile &t, const GuStage &g, i
     // One leaf at a time: hoisting the next leaf's loads and MFMAs above this
     // point multiplies the live registers.
     __builtin_amdgcn_sched_barrier(0);
-}
-
-// Leaves 2p and 2p+1 and their merge into the pairwise tree over v(0..31):
-// leaves are taken two at a time (a level-1 node) and merged upward like a
-// binary counter, so each level holds at most one pending left operand.
-// Levels 1-2 stay in registers; levels 3-4 (touched every 8, 16 leaves) wait
-// in LDS (`park`, 2 x 16 floats per lane of this wave).
-template<bool Full, bool Dbg>
-__device__ __forceinline__ void tree_step(const GuTile &t, const GuStage &g, float (*park)[16][64], int lane, int p,
-                                          float (&l1)[16], float (&l2)[16], float (&res)[16]) {
-    const int m = lane & 31, h = lane >> 5;
-    float w[16], x[16];
-    leaf_staged<Full, Dbg>(t, g, 2 * p, m, h, w);
-    leaf_staged<Full, Dbg>(t, g, 2 * p + 1, m, h, x);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = w[i] + x[i];
-    if ((p & 1) == 0) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) l1[i] = w[i];
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = l1[i] + w[i];
-    if ((p & 2) == 0) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) l2[i] = w[i];
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i] = l2[i] + w[i];
-    int lvl = 0;
-    for (; lvl < 2; ++lvl) {
-        if (((p >> (lvl + 2)) & 1) == 0) break;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) w[i] = park[lvl][i][lane] + w[i];
-    }
-    if (lvl < 2) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) park[lvl][i][lane] = w[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) res[i] = w[i];
-    }
-}
-
-template<bool Full, bool Dbg>
-__device__ __forceinline__ void fold_tree_staged(const GuTile &t, const GuStage &g, float (*park)[16][64], int lane,
-                                                 float (&res)[16]) {
-    float l1[16], l2[16];
-#pragma unroll 1
-    for (int p = 0; p < 16; ++p) tree_step<Full, Dbg>(t, g, park, lane, p, l1, l2, res);
 }
 
 // ---- H == 2048 (64 blocks): loads in groups of four leaves that use whole
@@ -732,7 +576,11 @@ __device__ __forceinline__ void leaf_grouped(const GuTile &t, const GuStage &g, 
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Tree merge of the level-1 node p (= w) as in tree_step.
+// Merge of the level-1 node p (= w, leaves 2p and 2p + 1) into the pairwise
+// tree over v(0..31), upward like a binary counter, so each level holds at
+// most one pending left operand.  Levels 1-2 stay in registers; levels 3-4
+// (touched every 8, 16 leaves) wait in LDS (`park`, 2 x 16 floats per lane of
+// this wave).
 __device__ __forceinline__ void tree_merge(float (*park)[16][64], int lane, int p, float (&w)[16], float (&l1)[16],
                                            float (&l2)[16], float (&res)[16]) {
     if ((p & 1) == 0) {
@@ -883,20 +731,22 @@ __device__ __forceinline__ void fold_tree_multi(const GuTile &t, float (*park)[1
 // are elements 16h..16h+15 of one Q8_1 block.  Units are ordered
 // (item, slice, sub) so the 4 tiles of an item that read the same weight rows
 // are adjacent on one XCD.
-// Fold: kFoldStaged (H < 2048), kFoldGrouped (H = 2048), kFoldGrouped96
-// (2048 < H <= 3072: the grouped leaves plus block kp + 64 in chain A;
-// 2560/640 4K Zipf layer 3.40 -> 2.83 ms with Q4_0 downs, 3.54 -> 2.98 ms
-// with Q4_1, against kFoldMulti), kFoldMulti (H > 3072); one instantiation
-// per shape keeps only that path's registers.
+// Rows of at most 64 blocks take k_gate_up_half (moe_half.hpp) instead; here
+// Fold is kFoldGrouped96 (2048 < H <= 3072: the grouped leaves plus block
+// kp + 64 in chain A; 2560/640 4K Zipf layer 3.40 -> 2.83 ms with Q4_0 downs,
+// 3.54 -> 2.98 ms with Q4_1, against kFoldMulti; the fp16-operand form with a
+// third block pair, two waves per SIMD at 63 KB of LDS, measured 3 % slower)
+// or kFoldMulti (H > 3072); one instantiation per shape keeps only that
+// path's registers.  The linear kernel below also takes kFoldStaged (< 64
+// blocks) and kFoldGrouped (64).
 enum { kFoldStaged = 0, kFoldGrouped = 1, kFoldMulti = 2, kFoldGrouped96 = 3 };
-constexpr int kGu96MaxBlocks = 96;
 
 template<int Fold, bool Dbg>
 __global__ __launch_bounds__(128, 2) void k_gate_up_mfma(FfnArgs a) {
     // Pending tree levels 3-4 per wave; after the tree the up wave's area
     // carries its result to the gate wave.
     __shared__ float park[2][2][16][64];
-    __shared__ uint4 d4_lds[2][Fold == kFoldGrouped96 ? kGu96MaxBlocks : kGuMaxBlocks][4];   // [mat][block][32 halfs]
+    __shared__ uint4 d4_lds[2][Fold == kFoldGrouped96 ? kGu96MaxBlocks : 1][4];   // [mat][block][32 halfs]
     float (*xch)[64] = park[1][0];
     const int mat = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int H = a.shape.H, I = a.shape.I, nb = H / 32, nbi = I / 32;
@@ -938,9 +788,9 @@ __global__ __launch_bounds__(128, 2) void k_gate_up_mfma(FfnArgs a) {
     // round trips overlap.
     const uint32_t w_off = static_cast<uint32_t>(prow) * row_bytes + 32u * 16u * h;
     uint4 wn[2] = {};
-    if constexpr (Fold == kFoldGrouped || Fold == kFoldGrouped96) half_load_w(t, w_off, 0, wn);
-    if constexpr (Fold != kFoldMulti) {
-        // Stage the tile's scales (both matrices) and its tokens' Q8 heads.
+    if constexpr (Fold == kFoldGrouped96) {
+        half_load_w(t, w_off, 0, wn);
+        // Stage the tile's scales (both matrices).
         // Scale group g (rows 8g..8g+7) of block b is one 16-byte chunk of the
         // [rows/8][blocks][8] plane and lands at halfs 8g..8g+7 of [mat][b].
         for (int c = threadIdx.x; c < 8 * nb; c += blockDim.x) {
@@ -950,9 +800,7 @@ __global__ __launch_bounds__(128, 2) void k_gate_up_mfma(FfnArgs a) {
         }
         __syncthreads();
         const GuStage g{reinterpret_cast<const uint32_t *>(&d4_lds[mat][0][0]), nullptr};
-        if constexpr (Fold == kFoldGrouped || Fold == kFoldGrouped96)
-            fold_tree_grouped<Dbg, Fold == kFoldGrouped96>(t, g, w_off, park[mat], lane, wn, res);
-        else fold_tree_staged<false, Dbg>(t, g, park[mat], lane, res);
+        fold_tree_grouped<Dbg, true>(t, g, w_off, park[mat], lane, wn, res);
     } else {
         fold_tree_multi<Dbg>(t, park[mat], lane, res);
     }
@@ -1623,25 +1471,9 @@ __global__ __launch_bounds__(512, 1) void k_down_mfma_pair(FfnArgs a) {
     }
 }
 
-// Upper bound on MFMA items: a group of n >= mfma_min pairs gives
-// ceil(n / 128) items, and at most min(Ep, pairs / mfma_min) groups qualify.
-size_t mfma_item_bound(const FfnArgs &a) {
-    const size_t P = static_cast<size_t>(a.pairs_bound);
-    const size_t G = std::min(P, static_cast<size_t>(a.shape.Ep));
-    const size_t big = a.mfma_min >= 1 ? std::min(G, P / static_cast<size_t>(a.mfma_min)) : G;
-    return std::max<size_t>(P / kMfmaTile + big, 1);
-}
-
 unsigned mfma_grid(const FfnArgs &a, int slices) {
     const size_t units = mfma_item_bound(a) * static_cast<size_t>(slices);
     const size_t round = 8 * static_cast<size_t>(kUnitChunk);
-    return static_cast<unsigned>((units + round - 1) / round * round);
-}
-
-// row_chunk_unit's grid: the units rounded up to whole rounds of 8 chunks.
-unsigned chunk_grid(const FfnArgs &a, int slices) {
-    const size_t units = mfma_item_bound(a) * static_cast<size_t>(slices);
-    const size_t round = 8 * static_cast<size_t>(kGuChunk);
     return static_cast<unsigned>((units + round - 1) / round * round);
 }
 
@@ -1853,21 +1685,14 @@ hipError_t launch_linear_mfma(const LinearMfmaArgs &a, hipStream_t s) {
 
 hipError_t launch_gate_up_mfma(const FfnArgs &a, hipStream_t s) {
     const bool dbg = a.middle_f32 || a.gate_dots || a.up_dots;
-    const unsigned grid = chunk_grid(a, a.shape.I / 32 * kSubs);
     const int nb = a.shape.H / 32;
-    if (nb == kGuMaxBlocks) {
-        if (dbg) k_gate_up_mfma<kFoldGrouped, true><<<grid, 128, 0, s>>>(a);
-        else k_gate_up_mfma<kFoldGrouped, false><<<grid, 128, 0, s>>>(a);
-    } else if (nb > kGuMaxBlocks && nb <= kGu96MaxBlocks) {
+    if (nb <= kHalfMaxBlocks) return launch_gate_up_half(a, s);
+    const unsigned grid = chunk_grid(a, a.shape.I / 32 * kSubs);
+    if (nb <= kGu96MaxBlocks) {
         if (dbg) k_gate_up_mfma<kFoldGrouped96, true><<<grid, 128, 0, s>>>(a);
         else k_gate_up_mfma<kFoldGrouped96, false><<<grid, 128, 0, s>>>(a);
-    } else if (nb < kGuMaxBlocks) {
-        if (dbg) k_gate_up_mfma<kFoldStaged, true><<<grid, 128, 0, s>>>(a);
-        else k_gate_up_mfma<kFoldStaged, false><<<grid, 128, 0, s>>>(a);
-    } else {
-        if (dbg) k_gate_up_mfma<kFoldMulti, true><<<grid, 128, 0, s>>>(a);
-        else k_gate_up_mfma<kFoldMulti, false><<<grid, 128, 0, s>>>(a);
-    }
+    } else if (dbg) k_gate_up_mfma<kFoldMulti, true><<<grid, 128, 0, s>>>(a);
+    else k_gate_up_mfma<kFoldMulti, false><<<grid, 128, 0, s>>>(a);
     return hipGetLastError();
 }
 

@@ -1,0 +1,54 @@
+"""GPU parity of the kernels on fp16 operands (csrc/moe_half.hpp) at the edges
+of their tiles: rows of 1..64 blocks (the 64-block form and the one that
+zero-fills missing blocks), an odd number of 32-row tiles (an idle second
+tile in the last workgroup), and token counts around the 32-token tiles.
+Every comparison is bit for bit: the kernels keep the reference's fp32 order.
+"""
+import numpy as np
+import pytest
+
+import moe_ffn
+import oracle as O
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu_ready():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    yield
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("H,I,columns", [
+    (2048, 32, 1), (2048, 96, 33), (2048, 64, 128), (2048, 160, 130),
+    (64, 96, 31), (960, 32, 32), (1088, 64, 64), (1984, 160, 97),
+])
+def test_gate_up_tile_edges(H, I, columns):
+    bank = W.q4_bank(2, hidden=H, intermediate=I, seed=H + I + columns)
+    L = moe_ffn.MoeLayer(H, I, 2, 1, False, columns, experts_q4=bank)
+    x = W.activations(columns, hidden=H, seed=columns)
+    x[columns // 2] *= 1e-3
+    xq = O.quantize_q8(x)
+    n = H // 32 * I * 18
+    blob = bank.reshape(2, -1)[1]
+    ref = O.expert_forward(blob[:n], blob[n:2 * n], blob[2 * n:], H, I, xq)
+    xd = torch.from_numpy(np.ascontiguousarray(xq).view(np.uint8).reshape(columns, -1)).to(DEV)
+    got = L.expert_gate_up(1, xd, columns, path=moe_ffn.PATH_MFMA)
+    torch.cuda.synchronize()
+    assert int(got["error"].cpu()[0]) == 0
+    assert np.array_equal(got["middle_q8"].cpu().numpy().reshape(-1),
+                          np.ascontiguousarray(ref["middle_q8"]).view(np.uint8).reshape(-1))
+    assert np.array_equal(got["middle"].cpu().numpy().view(np.uint32), ref["middle"].view(np.uint32))
+    # Without the fp32 middle: the kernel the forward runs.
+    mq = torch.empty_like(got["middle_q8"])
+    err = torch.zeros(1, dtype=torch.int32, device=DEV)
+    st = moe_ffn.library().moe_ffn_expert_gate_up(L.handle, 1, moe_ffn._ptr(xd), columns, None, moe_ffn._ptr(mq), None,
+                                                  None, moe_ffn.PATH_MFMA, moe_ffn._ptr(err), moe_ffn._stream(None))
+    torch.cuda.synchronize()
+    assert st == 0 and torch.equal(mq, got["middle_q8"])
+    L.close()
