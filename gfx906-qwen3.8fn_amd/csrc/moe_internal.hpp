@@ -208,6 +208,7 @@ hipError_t launch_gate_up_half_full(const FfnArgs &a, unsigned grid, hipStream_t
 struct LinearMfmaArgs {
     const uint8_t *codes;     // [Mp][nb][16 B]
     const uint16_t *scales;   // [Mp/8][nb][8]
+    const uint16_t *mins;     // Q4_1: same order as scales; Q4_0: null
     Act xq;                   // [N][nb] operand and head planes (xq.half, xq.heads), read when q8 is null
     const uint8_t *q8;        // canonical Q8_1 columns [N][nb][36 B] {d, s, qs[32]}, or null
     float *y;                 // [N][M]
@@ -217,6 +218,7 @@ struct LinearMfmaArgs {
     int waves;                // waves per workgroup: 4, or 8 (two tree nodes a wave)
 };
 hipError_t launch_linear_mfma(const LinearMfmaArgs &a, hipStream_t s);
+hipError_t launch_linear_mfma_q41(const LinearMfmaArgs &a, unsigned grid, hipStream_t s);   // moe_linear_q41.hip
 
 hipError_t launch_fold(const float *contributions, size_t token_stride, const float *weights, int k,
                        const int32_t *pos_of, const float *shared, size_t shared_stride,

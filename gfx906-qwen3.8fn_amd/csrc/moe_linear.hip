@@ -23,7 +23,7 @@
 // [rows/8][blocks][8], rows padded to a multiple of 32 with zero blocks, so a
 // lane's 8 row codes are eight 16-byte loads and its 8 scales one more.
 //
-// Wide batches (Q4_0, at least 32 columns and kMfmaMinOutputs outputs) go to
+// Wide batches (at least 32 columns and kMfmaMinOutputs outputs) go to
 // int8 MFMA instead (k_linear_mfma in moe_mfma.hip): the same fp32 order, with
 // the per-fragment integer dots from v_mfma_i32_32x32x16_i8.  forward_q8's
 // MFMA launch reads the caller's canonical blocks in place (any column
@@ -238,7 +238,15 @@ constexpr int kMfmaMinColumns = 32;        // one MFMA column tile
 // 10.6 against 8.65 / 8.87 / 9.0; 512 rows at 128 / 192 / 256 columns 6.35 /
 // 9.8 / 10.6 against 8.3 / 8.6 / 8.9; 2560 x 2560 at 48 columns 19.0 against
 // 13.3; 8192 rows at 32 columns 56.8 against 48.2).
+// Q4_1, vector / MFMA: 640 x 2560 at 48 / 128 / 1032 columns 14.8 / 31.9 / 232
+// against 9.6 / 11.5 / 35.1; 2560 x 640 at 64 / 128 / 1032
+// 10.7 / 19.7 / 115 against 16.1 / 17.0 / 39.7; 2048 x 2048 at 32 / 48 / 1032 9.2
+// / 12.9 / 146 against 11.9 / 11.9 / 50.5; 2048 x 512 at 128 / 256 9.6 / 14.3
+// against 11.8 / 12.7.  Rows of more than 96 blocks read every block's operands
+// on its own and pay later: 8192 x 2048 at 64 / 256 31.6 / 114 against 34.5 /
+// 63.4, 8192 x 8192 at 32 69.6 against 53.0.
 constexpr long kMfmaMinOutputs = 96 * 1024;
+constexpr long kMfmaMinOutputsQ41Long = 160 * 1024;
 
 bool aligned(const void *p, size_t a) { return p && reinterpret_cast<uintptr_t>(p) % a == 0; }
 size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -336,11 +344,11 @@ int moe_linear_bytes(const moe_linear *L, size_t *weight_bytes) {
 
 namespace {
 
-// MFMA for wide Q4_0 batches that fit the staging area (`capacity` columns).
+// MFMA for wide batches that fit the staging area (`capacity` columns).
 bool use_mfma_within(const moe_linear *L, int columns, int capacity) {
-    if (L->type != MOE_TYPE_Q4_0 || columns < kMfmaMinColumns || columns > capacity || L->mfma_mode == 0)
-        return false;
-    return L->mfma_mode == 1 || static_cast<long>(L->output) * columns >= kMfmaMinOutputs;
+    if (columns < kMfmaMinColumns || columns > capacity || L->mfma_mode == 0) return false;
+    const long least = L->type == MOE_TYPE_Q4_1 && L->nb > 96 ? kMfmaMinOutputsQ41Long : kMfmaMinOutputs;
+    return L->mfma_mode == 1 || static_cast<long>(L->output) * columns >= least;
 }
 bool use_mfma(const moe_linear *L, int columns) { return use_mfma_within(L, columns, L->max_columns); }
 
@@ -356,6 +364,7 @@ int launch_mfma(const moe_linear *L, moe::Act xq, const void *x_q8, int columns,
     moe::LinearMfmaArgs a{};
     a.codes = L->codes;
     a.scales = L->scales;
+    a.mins = L->mins;
     a.xq = xq;
     a.q8 = static_cast<const uint8_t *>(x_q8);
     a.y = y;
@@ -370,7 +379,7 @@ int launch_mfma(const moe_linear *L, moe::Act xq, const void *x_q8, int columns,
     // 10.5, 2048 x 512 at N = 320 / 512 10.2 / 10.9 -> 9.25 / 10.45, 2048 x
     // 1024 at N = 160 / 256 10.3 / 10.9 -> 9.35 / 10.5; larger grids lose:
     // 2048 x 2048 at N = 192 / 1032 16.0 / 54.5 -> 17.2 / 67.5).
-    a.waves = L->nb == 64 && static_cast<long>(a.row_tiles) * a.col_tiles <= 256 ? 8 : 4;
+    a.waves = L->type == MOE_TYPE_Q4_0 && L->nb == 64 && static_cast<long>(a.row_tiles) * a.col_tiles <= 256 ? 8 : 4;
     return moe::launch_linear_mfma(a, s);
 }
 

@@ -115,6 +115,7 @@ __device__ __forceinline__ float fma_mix_hi(uint32_t h2, float t, float acc) {
     return r;
 }
 
+constexpr uint32_t kNibbles = 0x0f0f0f0fu;
 constexpr int kGuMaxBlocks = 64, kGu96MaxBlocks = 96;
 
 // Upper bound on MFMA items: a group of n >= mfma_min pairs gives
