@@ -18,4 +18,14 @@ hipError_t launch_gate_up_half(const FfnArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t launch_linear_half(const LinearMfmaArgs &a, hipStream_t s) {
+    if (a.nb > kHalfMaxBlocks || a.mins || !(a.q8 || (a.xq.half && a.xq.heads))) return hipErrorInvalidValue;
+    const unsigned groups = static_cast<unsigned>((a.row_tiles + kHtWaves - 1) / kHtWaves);
+    const unsigned grid = (groups + 7u) / 8u * 8u * static_cast<unsigned>(a.col_tiles);
+    if (a.nb == kGuMaxBlocks) return launch_linear_half_full(a, grid, s);
+    if (a.q8) k_linear_half<false, true><<<grid, kHtThreads, 0, s>>>(a);
+    else k_linear_half<false, false><<<grid, kHtThreads, 0, s>>>(a);
+    return hipGetLastError();
+}
+
 }  // namespace moe

@@ -115,7 +115,8 @@ __device__ __forceinline__ uint2 codes_to_half(uint32_t c, bool high) {
 // (register v of lane half h, lane m: row 16h + v, token m).  Every wave of the
 // workgroup runs it (barriers); Full: 64 blocks, no block of a node is missing.
 // A missing block is staged as zeros (operand, head and scale), so its value
-// is the +0 of the reference's unused lane.  dots(p, i, q, F0, F1) receives the
+// is the +0 of the reference's unused lane; nodes and halves of nodes without
+// a block are left out (no lane value is -0, so adding +0 changes nothing).  dots(p, i, q, F0, F1) receives the
 // fragments of block 2p + i + 32q in the debug build.
 template<bool Full, bool Canon, bool Dbg, class Dots>
 __device__ __forceinline__ void half_tree(HalfLds &st, const HalfTile &t, int wave, float (&nd)[16], Dots &&dots) {
@@ -187,7 +188,14 @@ __device__ __forceinline__ void half_tree(HalfLds &st, const HalfTile &t, int wa
     float l1[16], l2[16];
 #pragma unroll 1
     for (int p = 0; p < 16; ++p) {
+        if (!Full && 2 * p >= nb) {   // uniform: no block left in this node or any later one
+#pragma unroll
+            for (int v = 0; v < 16; ++v) nd[v] = 0.0f;
+            merge_node(st.park[wave], lane, p, nd, l1, l2);
+            continue;
+        }
         const int buf = p & 1;
+        const bool both = Full || 2 * p + 32 < nb;   // uniform: the node has blocks 2p + 32, + 33
         const uint4 w[2] = {wn[0], wn[1]};
         fetch(p < 15 ? p + 1 : p);
         __builtin_amdgcn_sched_barrier(0);
@@ -215,10 +223,16 @@ __device__ __forceinline__ void half_tree(HalfLds &st, const HalfTile &t, int wa
                 const auto r = __builtin_amdgcn_permlane32_swap(wv[2 * f], wv[2 * f + 1], false, false);
                 const int sl = row ^ (4 * i + f);
                 const v16f Fa = frag_dot(r[0], (&st.x[buf][0][0][0])[sl]);
-                const v16f Fb = frag_dot(r[1], (&st.x[buf][1][0][0])[sl]);
+                if (both) {
+                    const v16f Fb = frag_dot(r[1], (&st.x[buf][1][0][0])[sl]);
 #pragma unroll
-                for (int v = 0; v < 16; ++v) u[f][v] = half_value(Fa[v], sa, da, v) + half_value(Fb[v], sb2, db, v);
-                if constexpr (Dbg) { ka[f] = Fa; kb[f] = Fb; }
+                    for (int v = 0; v < 16; ++v) u[f][v] = half_value(Fa[v], sa, da, v) + half_value(Fb[v], sb2, db, v);
+                    if constexpr (Dbg) kb[f] = Fb;
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) u[f][v] = half_value(Fa[v], sa, da, v);
+                }
+                if constexpr (Dbg) ka[f] = Fa;
             }
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
@@ -227,7 +241,7 @@ __device__ __forceinline__ void half_tree(HalfLds &st, const HalfTile &t, int wa
             }
             if constexpr (Dbg) {
                 dots(p, i, 0, ka[0], ka[1]);
-                dots(p, i, 1, kb[0], kb[1]);
+                if (both) dots(p, i, 1, kb[0], kb[1]);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -321,6 +335,50 @@ __global__ __launch_bounds__(kHtThreads, Dbg ? 2 : 3) void k_gate_up_half(FfnArg
         const int f = flags | (part == 0 ? q8.flags : 0);
         if (f) atomicOr(a.error, f);
     }
+}
+
+// Q4_0 linear on wide grids: 4 row tiles of 32 a workgroup against the same 32
+// columns.  Ids are XCD-aware: the column tiles of one row group run on one
+// XCD.  (The tree of one tile is one wave's work here; k_linear_mfma splits it
+// over a workgroup for grids that leave SIMDs idle.)
+template<bool Full, bool Canon>
+__global__ __launch_bounds__(kHtThreads, 3) void k_linear_half(LinearMfmaArgs a) {
+    __shared__ HalfLds st;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int id = static_cast<int>(blockIdx.x), local = id >> 3;
+    const int rg = (id & 7) + 8 * (local / a.col_tiles), c0 = local % a.col_tiles * kSub;
+    if (rg * kHtWaves >= a.row_tiles) return;   // uniform per workgroup (grid padded to 8 row groups)
+    const int rt = rg * kHtWaves + wave;
+    const bool active = rt < a.row_tiles;       // wave-uniform; an idle wave repeats the last tile
+    const int R0 = std::min(rt, a.row_tiles - 1) * 32, nb = a.nb;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint32_t row_bytes = static_cast<uint32_t>(nb) * 16u;
+    const auto column_row = [&](int i) {   // column c0 + i's first block (past N: the last column)
+        return static_cast<uint32_t>(std::min(c0 + i, a.N - 1)) * static_cast<uint32_t>(nb);
+    };
+    HalfTile t;
+    t.wr = buffer_rsrc(a.codes + static_cast<size_t>(R0) * row_bytes, 32u * row_bytes);
+    t.sr = buffer_rsrc(a.scales + static_cast<size_t>(R0) * nb, 32u * static_cast<uint32_t>(nb) * 2u);
+    const uint32_t blocks = static_cast<uint32_t>(a.N) * static_cast<uint32_t>(nb);
+    t.xr = Canon ? buffer_rsrc(a.q8, blocks * 36u) : buffer_rsrc(a.xq.half, blocks * 64u);
+    t.hr = Canon ? t.xr : buffer_rsrc(a.xq.heads, blocks * 4u);
+    t.x_base = column_row(tid >> 3) * HtXStride<Canon>;
+    t.h_base = column_row(tid & 31) * HtHStride<Canon>;
+    t.nb = nb;
+    float out[16];
+    half_tree<Full, Canon, false>(st, t, wave, out, [](int, int, int, v16f, v16f) {});
+    const int c = c0 + (lane & 31), row = R0 + 16 * (lane >> 5);
+    if (!active || c >= a.N) return;
+    float *yr = a.y + static_cast<size_t>(c) * a.M + row;
+    if (row + 16 <= a.M && (a.M & 3) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            reinterpret_cast<float4 *>(yr)[q] = make_float4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
+        return;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+        if (row + v < a.M) yr[v] = out[v];
 }
 
 }  // namespace

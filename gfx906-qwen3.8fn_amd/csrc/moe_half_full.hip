@@ -9,4 +9,10 @@ hipError_t launch_gate_up_half_full(const FfnArgs &a, unsigned grid, hipStream_t
     return hipGetLastError();
 }
 
+hipError_t launch_linear_half_full(const LinearMfmaArgs &a, unsigned grid, hipStream_t s) {
+    if (a.q8) k_linear_half<true, true><<<grid, kHtThreads, 0, s>>>(a);
+    else k_linear_half<true, false><<<grid, kHtThreads, 0, s>>>(a);
+    return hipGetLastError();
+}
+
 }  // namespace moe

@@ -209,7 +209,7 @@ struct LinearMfmaArgs {
     const uint8_t *codes;     // [Mp][nb][16 B]
     const uint16_t *scales;   // [Mp/8][nb][8]
     const uint16_t *mins;     // Q4_1: same order as scales; Q4_0: null
-    Act xq;                   // [N][nb] operand and head planes (xq.half, xq.heads), read when q8 is null
+    Act xq;                   // [N][nb] planes, read when q8 is null: heads and codes, or (launch_linear_half) half
     const uint8_t *q8;        // canonical Q8_1 columns [N][nb][36 B] {d, s, qs[32]}, or null
     float *y;                 // [N][M]
     int nb, M, N;
@@ -218,6 +218,10 @@ struct LinearMfmaArgs {
     int waves;                // waves per workgroup: 4, or 8 (two tree nodes a wave)
 };
 hipError_t launch_linear_mfma(const LinearMfmaArgs &a, hipStream_t s);
+// Q4_0 rows of at most 64 blocks on wide grids, on fp16 operands: xq.half or
+// canonical blocks (moe_half.hip, moe_half_full.hip).
+hipError_t launch_linear_half(const LinearMfmaArgs &a, hipStream_t s);
+hipError_t launch_linear_half_full(const LinearMfmaArgs &a, unsigned grid, hipStream_t s);
 hipError_t launch_linear_mfma_q41(const LinearMfmaArgs &a, unsigned grid, hipStream_t s);   // moe_linear_q41.hip
 
 hipError_t launch_fold(const float *contributions, size_t token_stride, const float *weights, int k,

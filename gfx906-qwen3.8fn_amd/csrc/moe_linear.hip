@@ -223,14 +223,24 @@ struct moe_linear {
     uint8_t *planes = nullptr;   // codes | scales | mins (one allocation)
     uint8_t *codes = nullptr;
     uint16_t *scales = nullptr, *mins = nullptr;
-    // apply's activation workspace, max_columns x nb x 36 B: canonical Q8_1
-    // blocks (narrow batches) or split planes (wide batches on MFMA).
+    // apply's activation workspace, max_columns x nb x workspace_block:
+    // canonical Q8_1 blocks (narrow batches) or planes (batches on MFMA).
     void *q8 = nullptr;
 };
 
 namespace {
 
 constexpr int kInvalid = hipErrorInvalidValue;
+constexpr size_t kHalfPlaneBytes = 68;     // per block: 64 B of fp16 operands, 4 B of head
+// Workgroups (128 rows x 32 columns) from which the fp16-operand kernel wins:
+// its tile is one wave's 32 leaves (25 us alone), so it needs two to three
+// workgroups a CU.  us, k_linear_mfma / k_linear_half, rows of 64 blocks: 528
+// groups (2048 x 2048 at 1,032 columns) 53.3 / 55.0, 752 (at 1,500) 74.4 / 61.5,
+// 1,024 (2048 x 8192 at 512) 87.6 / 74.4; 32 blocks: 1,504 (1024 x 4096 at 1,500)
+// 82.7 / 71.8; rows of 20 blocks lose (660 groups 35.3 / 46.7): they keep the
+// split kernel, as all below 32 do.
+constexpr long kHalfMinGroups = 700;
+constexpr int kHalfMinBlocks = 32;
 constexpr int kMfmaMinColumns = 32;        // one MFMA column tile
 // Outputs (rows x columns) from which the MFMA kernel beats the vector one
 // (MI355X, cold weights, vector / MFMA us with the per-launch vector plans
@@ -256,6 +266,16 @@ void release(moe_linear *L) {
     if (L->planes) (void)hipFree(L->planes);
     if (L->q8) (void)hipFree(L->q8);
     delete L;
+}
+
+// Matrices the fp16-operand kernel takes.
+bool half_rows(const moe_linear *L) {
+    return L->type == MOE_TYPE_Q4_0 && L->nb >= kHalfMinBlocks && L->nb <= moe::kHalfMaxBlocks;
+}
+
+// Bytes per block of apply's workspace: the largest staging its matrix can use.
+size_t workspace_block(const moe_linear *L) {
+    return half_rows(L) ? kHalfPlaneBytes : 36;
 }
 
 int block_bytes(int type) { return type == MOE_TYPE_Q4_1 ? 20 : 18; }
@@ -301,7 +321,7 @@ int moe_linear_create(int type, int input, int output, int max_columns, const vo
     L->codes = L->planes;
     L->scales = reinterpret_cast<uint16_t *>(L->planes + code_bytes);
     L->mins = type == MOE_TYPE_Q4_1 ? reinterpret_cast<uint16_t *>(L->planes + code_bytes + scale_bytes) : nullptr;
-    if (max_columns > 0 && (r = hipMalloc(&L->q8, static_cast<size_t>(max_columns) * L->nb * 36)) != hipSuccess) {
+    if (max_columns > 0 && (r = hipMalloc(&L->q8, static_cast<size_t>(max_columns) * L->nb * workspace_block(L))) != hipSuccess) {
         release(L);
         return r;
     }
@@ -352,14 +372,22 @@ bool use_mfma_within(const moe_linear *L, int columns, int capacity) {
 }
 bool use_mfma(const moe_linear *L, int columns) { return use_mfma_within(L, columns, L->max_columns); }
 
-// Split Q8 planes for `columns` columns at `base` (codes, then heads).
-moe::Act staging_planes(const moe_linear *L, void *base_ptr, int columns) {
-    auto *base = static_cast<uint8_t *>(base_ptr);
-    return moe::Act{base, reinterpret_cast<uint32_t *>(base + static_cast<size_t>(columns) * L->nb * 32)};
+// Grids of at least kHalfMinGroups workgroups take the fp16-operand kernel.
+bool use_half(const moe_linear *L, int columns) {
+    const long groups = static_cast<long>((L->Mp / 32 + 3) / 4) * ((columns + 31) / 32);
+    return half_rows(L) && groups >= kHalfMinGroups;
 }
-moe::Act workspace_planes(const moe_linear *L, int columns) { return staging_planes(L, L->q8, columns); }
 
-// x_q8: canonical Q8_1 columns read in place, else the split planes xq.
+// Planes for `columns` columns at `base_ptr`: fp16 operands (half) or codes,
+// then heads.
+moe::Act staging_planes(const moe_linear *L, void *base_ptr, int columns, bool half) {
+    auto *base = static_cast<uint8_t *>(base_ptr);
+    const size_t blocks = static_cast<size_t>(columns) * L->nb;
+    if (half) return moe::Act{nullptr, reinterpret_cast<uint32_t *>(base + blocks * 64), reinterpret_cast<uint16_t *>(base)};
+    return moe::Act{base, reinterpret_cast<uint32_t *>(base + blocks * 32)};
+}
+
+// x_q8: canonical Q8_1 columns read in place, else the planes xq.
 int launch_mfma(const moe_linear *L, moe::Act xq, const void *x_q8, int columns, float *y, hipStream_t s) {
     moe::LinearMfmaArgs a{};
     a.codes = L->codes;
@@ -373,6 +401,7 @@ int launch_mfma(const moe_linear *L, moe::Act xq, const void *x_q8, int columns,
     a.N = columns;
     a.row_tiles = L->Mp / 32;
     a.col_tiles = (columns + 31) / 32;
+    if (use_half(L, columns)) return moe::launch_linear_half(a, s);
     // 8-wave workgroups (two tree nodes a wave) for 64-block rows where the
     // 4-wave grid gives at most one workgroup per CU (us, 4 -> 8 waves,
     // forward_q8 cold: 2048 x 2048 at N = 80 / 128 10.5 / 11.1 -> 9.45 /
@@ -505,7 +534,7 @@ int moe_linear_apply(moe_linear *L, const float *x, int columns, float *y, int *
         return kInvalid;
     const auto s = static_cast<hipStream_t>(stream);
     if (use_mfma(L, columns)) {
-        const moe::Act xq = workspace_planes(L, columns);
+        const moe::Act xq = staging_planes(L, L->q8, columns, use_half(L, columns));
         const hipError_t r = moe::launch_quantize_planes(x, xq, L->input, columns, error, s);
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
@@ -517,8 +546,7 @@ int moe_linear_apply(moe_linear *L, const float *x, int columns, float *y, int *
 
 int moe_linear_apply_noalloc(moe_linear *L, const float *x, int columns, float *y, int *error, void *stream) {
     if (!L || !aligned(x, 4) || !aligned(y, 4) || !aligned(error, 4) || columns < 1) return kInvalid;
-    // The staging (canonical Q8_1 blocks, or the MFMA kernel's split planes:
-    // 36 bytes per block either way) must fit the static array.
+    // The canonical Q8_1 blocks must fit the static array.
     if (static_cast<size_t>(columns) * L->nb * 36 > kNoallocScratchBytes) return kInvalid;
     int device = -1;
     if (hipGetDevice(&device) != hipSuccess || device != L->device) return kInvalid;
@@ -530,15 +558,18 @@ int moe_linear_apply_noalloc(moe_linear *L, const float *x, int columns, float *
         ~Release() { flag.store(0, std::memory_order_release); }
     } release_busy{scratch_busy[device]};
     const auto s = static_cast<hipStream_t>(stream);
-    const int capacity = static_cast<int>(kNoallocScratchBytes / (static_cast<size_t>(L->nb) * 36));
-    if (use_mfma_within(L, columns, capacity)) {
-        const moe::Act xq = staging_planes(L, ws, columns);
+    const bool mfma = use_mfma_within(L, columns, 65536), half = mfma && use_half(L, columns);
+    if (mfma && static_cast<size_t>(columns) * L->nb * (half ? kHalfPlaneBytes : 36) <= kNoallocScratchBytes) {
+        const moe::Act xq = staging_planes(L, ws, columns, half);
         const hipError_t r = moe::launch_quantize_planes(x, xq, L->input, columns, error, s);
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
     }
     const hipError_t r = moe::launch_quantize_canonical(x, ws, L->input, columns, error, s);
     if (r != hipSuccess) return r;
+    // Batches whose operand planes outgrow the array: canonical blocks, which
+    // the MFMA kernels read as well.
+    if (mfma) return launch_mfma(L, moe::Act{}, ws, columns, y, s);
     return launch_vector(L, ws, columns, y, s);
 }
 

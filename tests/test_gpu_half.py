@@ -52,3 +52,27 @@ def test_gate_up_tile_edges(H, I, columns):
     torch.cuda.synchronize()
     assert st == 0 and torch.equal(mq, got["middle_q8"])
     L.close()
+
+
+@pytest.mark.parametrize("K,M,N", [(1024, 2820, 1000), (2048, 2820, 1000), (1984, 2816, 1001)])
+def test_linear_wide_grid_matches_vector(K, M, N, monkeypatch):
+    """Grids wide enough for the fp16-operand linear (canonical input, planes,
+    and both stagings of the no-allocation call) against the vector kernel,
+    which the oracle pins: ragged last rows and columns."""
+    w = W.q4_blocks(M * K // 32, np.random.default_rng(K + M)).reshape(-1)
+    x = torch.from_numpy(W.activations(N, hidden=K, seed=N)).to(DEV)
+    monkeypatch.setenv("MOE_LINEAR_MFMA", "0")
+    V = moe_ffn.MoeLinear(moe_ffn.TYPE_Q4_0, K, M, w, max_columns=N)
+    monkeypatch.delenv("MOE_LINEAR_MFMA")
+    L = moe_ffn.MoeLinear(moe_ffn.TYPE_Q4_0, K, M, w, max_columns=N)
+    q8, _ = moe_ffn.quantize_q8_1(x)
+    ref = V.forward_q8(q8, N).view(torch.int32)
+    assert torch.equal(L.forward_q8(q8, N).view(torch.int32), ref)
+    assert torch.equal(L.apply(x)[0].view(torch.int32), ref)
+    y = torch.empty((N, M), dtype=torch.float32, device=DEV)
+    e = torch.zeros(1, dtype=torch.int32, device=DEV)
+    L.apply_noalloc(x, y, e)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int32), ref) and int(e.cpu()[0]) == 0
+    V.close()
+    L.close()
