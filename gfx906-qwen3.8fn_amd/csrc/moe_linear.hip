@@ -171,6 +171,113 @@ __global__ __launch_bounds__(64, ROWS == 4 ? (G == 4 ? 3 : 4) : 2) void k_linear
     }
 }
 
+// The vector kernel from fp32 columns, for the few columns of a decode step:
+// a workgroup of 4 waves quantizes all G columns into LDS itself (4 lanes a
+// block, the bytes of k_quantize) while its first weights are in flight, then
+// each wave takes 4 rows as k_linear does.  Bound by latency: a launch of its
+// own for the quantisation costs about 2 us, repeating it in every workgroup
+// about 1.1 us per 64 blocks (2048 x 2048 at one column 4.93 -> 3.32 us).
+template<bool Q41, int G>
+__global__ __launch_bounds__(256) void k_linear_fp32(LinearArgs a, const float *__restrict__ x, int *error) {
+    constexpr int ROWS = 4;
+    extern __shared__ uint32_t lds[];
+    const int nb = a.nb, blocks = G * nb, slots = (nb + 63) / 64;
+    uint32_t *codes = lds;                 // [G][nb][8]
+    uint32_t *heads = lds + blocks * 8;    // [G][nb]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = (static_cast<int>(blockIdx.x) * 4 + wave) * ROWS;
+    const bool active = row0 < a.slices * ROWS;   // wave-uniform
+    const uint32_t row_bytes = static_cast<uint32_t>(nb) * 16u;
+    const int arow = active ? row0 : 0;
+    const auto wr = buffer_rsrc(a.codes + static_cast<size_t>(arow) * row_bytes, ROWS * row_bytes);
+    const size_t g0 = static_cast<size_t>(arow & ~7);
+    const uint32_t shalf = static_cast<uint32_t>(arow & 4) * 2u;
+    const auto sr = buffer_rsrc(a.scales + g0 * nb, row_bytes);
+    const auto mr = buffer_rsrc(Q41 ? a.mins + g0 * nb : a.scales, row_bytes);
+    // This pass's 64 blocks: x first, so that waiting for it never waits
+    // behind the weights.
+    const int part = lane >> 4, qb = wave * 16 + (lane & 15);
+    const auto xr = buffer_rsrc(x, static_cast<uint32_t>(blocks) * 128u);
+    uint4 xa = buffer_load16(xr, static_cast<uint32_t>(qb) * 128u + 32u * part, 0);
+    uint4 xb = buffer_load16(xr, static_cast<uint32_t>(qb) * 128u + 32u * part, 16);
+    uint4 w[ROWS];
+    uint32_t dw[2], mw[2] = {};
+    const auto load_slot = [&](int i) {   // lanes past the row end load block 0 and keep their accumulators
+        const int k = lane + 64 * i;
+        const uint32_t kk = k < nb ? static_cast<uint32_t>(k) : 0u;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) w[r] = buffer_load16(wr, kk * 16u, r * row_bytes);
+        const auto dp = __builtin_amdgcn_raw_buffer_load_b64(sr, kk * 16u + shalf, 0, 0);
+        dw[0] = dp[0]; dw[1] = dp[1];
+        if constexpr (Q41) {
+            const auto mp = __builtin_amdgcn_raw_buffer_load_b64(mr, kk * 16u + shalf, 0, 0);
+            mw[0] = mp[0]; mw[1] = mp[1];
+        }
+    };
+    load_slot(0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int b0 = 0; b0 < blocks; b0 += 64) {   // uniform
+        float v[8] = {__uint_as_float(xa.x), __uint_as_float(xa.y), __uint_as_float(xa.z), __uint_as_float(xa.w),
+                      __uint_as_float(xb.x), __uint_as_float(xb.y), __uint_as_float(xb.z), __uint_as_float(xb.w)};
+        const int b = b0 + qb;
+        const uint32_t next = static_cast<uint32_t>(b + 64) * 128u + 32u * part;   // past the columns: reads zeros
+        xa = buffer_load16(xr, next, 0);
+        xb = buffer_load16(xr, next, 16);
+        const Q8Part<4> q = quantize_part<4>(v);
+        if (b < blocks) {
+            *reinterpret_cast<uint2 *>(codes + b * 8 + 2 * part) = make_uint2(q.codes[0], q.codes[1]);
+            if (part == 0) {
+                heads[b] = q.head;
+                if (blockIdx.x == 0 && q.flags) atomicOr(error, q.flags);
+            }
+        }
+    }
+    __syncthreads();
+    if (!active) return;
+    float acc[G][ROWS][2] = {};
+    for (int i = 0; i < slots; ++i) {   // uniform
+        if (i > 0) load_slot(i);
+        const int k = lane + 64 * i;
+        const bool has = k < nb;
+        const int kk = has ? k : 0;
+        float d4[ROWS], m4[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            d4[r] = h2f(dw[r >> 1] >> (16 * (r & 1)));
+            m4[r] = Q41 ? h2f(mw[r >> 1] >> (16 * (r & 1))) : 0.0f;
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const uint32_t head = heads[g * nb + kk];
+            const uint4 *cp = reinterpret_cast<const uint4 *>(codes + (g * nb + kk) * 8);
+            const uint4 x0 = cp[0], x1 = cp[1];
+            const float d8 = h2f(head), s8 = h2f(head >> 16), c4 = -4.0f * s8;
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                int f[2];
+                fragment_dots(w[r], x0, x1, f[0], f[1]);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    float v;
+                    if constexpr (Q41) {
+                        const float dd = h2f(f2h(d4[r] * d8)), hm = h2f(f2h(m4[r] * s8)) * 0.5f;
+                        v = acc[g][r][q] + fmaf(static_cast<float>(f[q]), dd, hm);
+                    } else {
+                        v = fmaf(d4[r], fmaf(static_cast<float>(f[q]), d8, c4), acc[g][r][q]);
+                    }
+                    acc[g][r][q] = has ? v : acc[g][r][q];
+                }
+            }
+        }
+    }
+    const int row = row0 + 2 * ((lane >> 5) & 1) + (lane & 1);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const float v = fold_rows4(acc[g], lane);
+        if ((lane & 30) == 0 && row < a.M) a.y[static_cast<size_t>(g) * a.M + row] = v;
+    }
+}
+
 }  // namespace
 }  // namespace moe
 
@@ -279,6 +386,46 @@ size_t workspace_block(const moe_linear *L) {
 }
 
 int block_bytes(int type) { return type == MOE_TYPE_Q4_1 ? 20 : 18; }
+
+// Columns x blocks up to which a batch quantizes inside the vector kernel
+// (k_linear_fp32): each further pass of 64 blocks costs every workgroup about
+// 1.1 us, the launch it saves about 2.  apply, us, two launches / one: 64 blocks
+// 2048 x 2048 at one column 4.93 / 3.32, 2048 x 512 4.41 / 3.17, 2048 x 8192
+// 5.93 / 5.40; 80 blocks 2560 x 640 4.85 / 4.36, Q4_1 2560 x 2560 5.49 / 5.19,
+// Q4_1 640 x 2560 at 4 columns 5.09 / 5.08; 128 blocks, two columns of 2048:
+// 2048 rows 4.81 / 4.49, 512 4.39 / 4.43, 8192 6.68 / 7.09; 256 blocks, 8192 x
+// 8192 at one 11.3 / 13.5.
+constexpr int kFusedBlocks = 80;
+bool use_fused(const moe_linear *L, int columns) {
+    return columns <= 4 && columns * L->nb <= kFusedBlocks && L->vector_g == 0 && L->vector_rows == 0;
+}
+
+template<bool Q41>
+int launch_fused_t(const moe::LinearArgs &a, const float *x, int *error, unsigned grid, hipStream_t s) {
+    const unsigned lds = static_cast<unsigned>(a.N * a.nb) * 36u;
+    switch (a.N) {
+    case 1: moe::k_linear_fp32<Q41, 1><<<grid, 256, lds, s>>>(a, x, error); break;
+    case 2: moe::k_linear_fp32<Q41, 2><<<grid, 256, lds, s>>>(a, x, error); break;
+    case 3: moe::k_linear_fp32<Q41, 3><<<grid, 256, lds, s>>>(a, x, error); break;
+    case 4: moe::k_linear_fp32<Q41, 4><<<grid, 256, lds, s>>>(a, x, error); break;
+    default: return kInvalid;
+    }
+    return hipGetLastError();
+}
+
+int launch_fused(const moe_linear *L, const float *x, int columns, float *y, int *error, hipStream_t s) {
+    moe::LinearArgs a{};
+    a.codes = L->codes;
+    a.scales = L->scales;
+    a.mins = L->mins;
+    a.y = y;
+    a.nb = L->nb;
+    a.M = L->output;
+    a.N = columns;
+    a.slices = (L->output + 3) / 4;
+    const unsigned grid = static_cast<unsigned>((a.slices + 3) / 4);
+    return L->type == MOE_TYPE_Q4_1 ? launch_fused_t<true>(a, x, error, grid, s) : launch_fused_t<false>(a, x, error, grid, s);
+}
 
 }  // namespace
 
@@ -539,6 +686,7 @@ int moe_linear_apply(moe_linear *L, const float *x, int columns, float *y, int *
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
     }
+    if (use_fused(L, columns)) return launch_fused(L, x, columns, y, error, s);
     const hipError_t r = moe::launch_quantize_canonical(x, L->q8, L->input, columns, error, s);
     if (r != hipSuccess) return r;
     return moe_linear_forward_q8(L, L->q8, columns, y, stream);
@@ -565,6 +713,7 @@ int moe_linear_apply_noalloc(moe_linear *L, const float *x, int columns, float *
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
     }
+    if (use_fused(L, columns)) return launch_fused(L, x, columns, y, error, s);
     const hipError_t r = moe::launch_quantize_canonical(x, ws, L->input, columns, error, s);
     if (r != hipSuccess) return r;
     // Batches whose operand planes outgrow the array: canonical blocks, which
