@@ -6,7 +6,7 @@
 namespace moe {
 
 hipError_t launch_gate_up_half(const FfnArgs &a, hipStream_t s) {
-    if (!a.xq.half) return hipErrorInvalidValue;
+    if (!a.xhalf) return hipErrorInvalidValue;
     const bool dbg = a.middle_f32 || a.gate_dots || a.up_dots;
     const int nb = a.shape.H / 32;
     const unsigned grid = chunk_grid(a, (a.shape.I / 32 + kGuTiles - 1) / kGuTiles * kSubs, kGuChunkRows / kGuTiles);

@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kHtThreads, Dbg ? 2 : 3) void k_gate_up_half(FfnArg
     HalfTile t;
     t.wr = buffer_rsrc((mat ? a.bank.up_codes : a.bank.gate_codes) + rbase * row_bytes, 32u * row_bytes);
     t.sr = buffer_rsrc((mat ? a.bank.up_scales : a.bank.gate_scales) + rbase * nb, 32u * static_cast<uint32_t>(nb) * 2u);
-    t.xr = buffer_rsrc(a.xq.half, static_cast<uint32_t>(a.tokens) * static_cast<uint32_t>(nb) * 64u);
+    t.xr = buffer_rsrc(a.xhalf, static_cast<uint32_t>(a.tokens) * static_cast<uint32_t>(nb) * 64u);
     t.hr = buffer_rsrc(a.xq.heads, static_cast<uint32_t>(a.tokens) * static_cast<uint32_t>(nb) * 4u);
     t.x_base = token_row(tid >> 3) * 64u;
     t.h_base = token_row(tid & 31) * 4u;

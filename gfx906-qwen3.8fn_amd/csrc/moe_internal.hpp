@@ -95,6 +95,9 @@ struct RouteOut {
 struct Act {               // split-plane Q8 rows
     uint8_t *codes;        // [rows][blocks][32]
     uint32_t *heads;       // [rows][blocks]
+};
+// Q8 rows as a quantiser writes them: the planes that are there.
+struct ActOut : Act {
     uint16_t *half = nullptr;   // [rows][blocks][32] fp16 MFMA operands (half_slot), or null: not written
 };
 
@@ -121,9 +124,9 @@ __host__ __device__ constexpr int half_slot(int e) {
 // enqueue; argument validation is done by the callers in moe_layer.hip.
 hipError_t launch_quantize_canonical(const float *x, void *q8, int width, int columns, int *error,
                                      hipStream_t s);
-hipError_t launch_quantize_planes(const float *x, Act out, int width, int columns, int *error,
+hipError_t launch_quantize_planes(const float *x, ActOut out, int width, int columns, int *error,
                                   hipStream_t s);
-hipError_t launch_canonical_to_planes(const void *q8, Act out, int blocks, hipStream_t s);
+hipError_t launch_canonical_to_planes(const void *q8, ActOut out, int blocks, hipStream_t s);
 hipError_t launch_planes_to_canonical(Act in, void *q8, int blocks, hipStream_t s);
 
 // Weight planes of one matrix kind (codes / scales = plane bases).  The call
@@ -143,7 +146,7 @@ hipError_t launch_synthetic_weights(uint8_t *codes, uint16_t *scales, uint16_t *
 // Quantize x into `xq` and group routes (tokens <= kSmallGroupTokens path or
 // the multi-kernel path).  mfma_min = smallest group that goes to MFMA (0 = never).
 hipError_t launch_prepare(const float *x, const int32_t *ids, const float *weights, int tokens,
-                          Shape shape, Act xq, RouteOut routes, int mfma_min, int *error,
+                          Shape shape, ActOut xq, RouteOut routes, int mfma_min, int *error,
                           hipStream_t s);
 
 // Single-expert stage setup: pairs 0..columns-1 = tokens 0..columns-1 of
@@ -165,7 +168,7 @@ struct FfnArgs {
     float *middle_f32; // optional [pairs][I]
     int32_t *gate_dots, *up_dots, *down_dots;  // optional per-block dots [pair][rows][blocks]
     int *error;
-    int cu_count;      // compute units of the device (persistent grids)
+    const uint16_t *xhalf;   // fp16 operand plane of xq's rows, or null
 };
 
 // Ungrouped decode path (few tokens, mostly one token per expert): work is
@@ -209,7 +212,7 @@ struct LinearMfmaArgs {
     const uint8_t *codes;     // [Mp][nb][16 B]
     const uint16_t *scales;   // [Mp/8][nb][8]
     const uint16_t *mins;     // Q4_1: same order as scales; Q4_0: null
-    Act xq;                   // [N][nb] planes, read when q8 is null: heads and codes, or (launch_linear_half) half
+    ActOut xq;                // [N][nb] planes, read when q8 is null: heads and codes, or (launch_linear_half) half
     const uint8_t *q8;        // canonical Q8_1 columns [N][nb][36 B] {d, s, qs[32]}, or null
     float *y;                 // [N][M]
     int nb, M, N;

@@ -58,7 +58,7 @@ __device__ __forceinline__ void store_half_part(uint16_t *half, size_t block, in
 }
 
 // The planes that are there: codes, the fp16 operands, heads.
-__device__ __forceinline__ void store_planes(const Act &out, size_t block, int part, const Q8Part<4> &q, int *error) {
+__device__ __forceinline__ void store_planes(const ActOut &out, size_t block, int part, const Q8Part<4> &q, int *error) {
     if (out.codes) *reinterpret_cast<uint2 *>(out.codes + block * 32 + 8 * part) = make_uint2(q.codes[0], q.codes[1]);
     if (out.half) store_half_part(out.half, block, part, q.codes);
     if (part == 0) {
@@ -70,7 +70,7 @@ __device__ __forceinline__ void store_planes(const Act &out, size_t block, int p
 // One element per lane, a block per 32 lanes: short batches, whose time is
 // one wave's latency.
 template<bool Canonical>
-__global__ __launch_bounds__(256) void k_quantize_short(const float *__restrict__ x, Act out, size_t elements, int *error) {
+__global__ __launch_bounds__(256) void k_quantize_short(const float *__restrict__ x, ActOut out, size_t elements, int *error) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= elements) return;   // elements is a multiple of 32: whole groups exit together
     const Q8Lane q = quantize32(x[i]);
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void k_quantize_short(const float *__restrict_
 // butterflies, here a quarter as many a value).  Canonical, width 2048, us, one
 // element a lane -> eight: 1,032 columns 7.7 -> 4.2, 4,096 25.0 -> 9.9.
 template<bool Canonical>
-__global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ x, Act out, size_t elements, int *error) {
+__global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ x, ActOut out, size_t elements, int *error) {
     quantize_group(x, static_cast<size_t>(blockIdx.x) * 64, elements, [&](size_t block, int part, const Q8Part<4> &q) {
         if constexpr (Canonical) {
             uint32_t *dst = reinterpret_cast<uint32_t *>(out.codes + block * 36);
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ x, A
     });
 }
 
-__global__ __launch_bounds__(256) void k_canonical_to_planes(const uint8_t *q8, Act out, size_t blocks) {
+__global__ __launch_bounds__(256) void k_canonical_to_planes(const uint8_t *q8, ActOut out, size_t blocks) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= blocks * 9) return;
     const size_t b = i / 9, w = i % 9;
@@ -354,7 +354,7 @@ __device__ void build_items(const GroupParams &p, const int32_t *cnt, const int3
 
 // Small path: block 0 groups (bitmaps in LDS), blocks 1.. quantize x.
 __global__ __launch_bounds__(1024) void k_prepare_small(GroupParams p, const float *__restrict__ x,
-                                                        Act xq, size_t q_elements) {
+                                                        ActOut xq, size_t q_elements) {
     extern __shared__ uint32_t lds[];
     if (blockIdx.x > 0) {
         const size_t i = static_cast<size_t>(blockIdx.x - 1) * blockDim.x + threadIdx.x;
@@ -494,7 +494,7 @@ __device__ int weight_flags(const GroupParams &p, int t0) {
 // the rest quantize x.  The bitmap is [W][Ep] (word-major) so the
 // per-expert prefix kernel reads it coalesced.
 __global__ __launch_bounds__(256) void k_mark_quantize(GroupParams p, int mark_blocks,
-                                                       const float *__restrict__ x, Act xq,
+                                                       const float *__restrict__ x, ActOut xq,
                                                        size_t q_elements) {
     extern __shared__ uint32_t lds[];
     if (static_cast<int>(blockIdx.x) < mark_blocks) {
@@ -1975,7 +1975,7 @@ namespace {
 constexpr size_t kQuantizeShort = size_t{256} * 2048;
 
 template<bool Canonical>
-void launch_quantize(const float *x, Act out, size_t n, int *error, hipStream_t s) {
+void launch_quantize(const float *x, ActOut out, size_t n, int *error, hipStream_t s) {
     if (n < kQuantizeShort) k_quantize_short<Canonical><<<blocks_for(n, 256), 256, 0, s>>>(x, out, n, error);
     else k_quantize<Canonical><<<blocks_for(n, 2048), 256, 0, s>>>(x, out, n, error);
 }
@@ -1984,18 +1984,18 @@ void launch_quantize(const float *x, Act out, size_t n, int *error, hipStream_t 
 hipError_t launch_quantize_canonical(const float *x, void *q8, int width, int columns, int *error,
                                      hipStream_t s) {
     const size_t n = static_cast<size_t>(width) * columns;
-    launch_quantize<true>(x, Act{static_cast<uint8_t *>(q8), nullptr}, n, error, s);
+    launch_quantize<true>(x, ActOut{{static_cast<uint8_t *>(q8), nullptr}}, n, error, s);
     return hipGetLastError();
 }
 
-hipError_t launch_quantize_planes(const float *x, Act out, int width, int columns, int *error,
+hipError_t launch_quantize_planes(const float *x, ActOut out, int width, int columns, int *error,
                                   hipStream_t s) {
     const size_t n = static_cast<size_t>(width) * columns;
     launch_quantize<false>(x, out, n, error, s);
     return hipGetLastError();
 }
 
-hipError_t launch_canonical_to_planes(const void *q8, Act out, int blocks, hipStream_t s) {
+hipError_t launch_canonical_to_planes(const void *q8, ActOut out, int blocks, hipStream_t s) {
     const size_t n = static_cast<size_t>(blocks) * 9;
     k_canonical_to_planes<<<blocks_for(n, 256), 256, 0, s>>>(static_cast<const uint8_t *>(q8), out,
                                                               static_cast<size_t>(blocks));
@@ -2054,7 +2054,7 @@ hipError_t launch_fill_u32(uint32_t *p, uint32_t value, size_t count, hipStream_
 }
 
 hipError_t launch_prepare(const float *x, const int32_t *ids, const float *weights, int tokens, Shape shape,
-                          Act xq, RouteOut routes, int mfma_min, int *error, hipStream_t s) {
+                          ActOut xq, RouteOut routes, int mfma_min, int *error, hipStream_t s) {
     GroupParams p{ids, weights, tokens, shape, routes, mfma_min, error};
     // Grouping alone (x == nullptr, as moe_ffn_group_routes calls it) launches
     // no quantization blocks: they would read x.

@@ -38,6 +38,7 @@ struct moe_ffn_layer {
     void *ws_mem = nullptr;
     size_t ws_bytes = 0;
     Act xq{}, mq{};
+    uint16_t *xhalf = nullptr;   // fp16 operand plane of xq (rows of at most kHalfMaxBlocks blocks)
     RouteOut routes{};
     float *contrib = nullptr;
     // Error word of the diagnostics (debug_last / last_stats re-group a
@@ -62,7 +63,6 @@ struct moe_ffn_layer {
     int active_mfma_min = 12;   // mfma_min of the current / last forward
     int decode_mode = -1; // ungrouped decode path: -1 auto, 0 never, 1 whenever shapes allow
     bool last_decode = false;
-    int cu_count = 256;   // compute units of the device
     int last_tokens = 0;
     // Inputs of the last forward (for moe_ffn_replay_stage).
     const float *last_x = nullptr, *last_weights = nullptr, *last_shared_gate = nullptr;
@@ -167,8 +167,8 @@ int finish_create(moe_ffn_layer *L) {
     if (hipMalloc(&L->ws_mem, w.total) != hipSuccess) return hipErrorOutOfMemory;
     L->ws_bytes = w.total;
     auto *b = static_cast<uint8_t *>(L->ws_mem);
-    L->xq = Act{b + w.xq_codes, reinterpret_cast<uint32_t *>(b + w.xq_heads),
-                reinterpret_cast<uint16_t *>(b + w.xq_half)};
+    L->xq = Act{b + w.xq_codes, reinterpret_cast<uint32_t *>(b + w.xq_heads)};
+    L->xhalf = L->shape.H / 32 <= moe::kHalfMaxBlocks ? reinterpret_cast<uint16_t *>(b + w.xq_half) : nullptr;
     L->mq = Act{b + w.mq_codes, reinterpret_cast<uint32_t *>(b + w.mq_heads)};
     L->routes.pair_token = reinterpret_cast<int32_t *>(b + w.pair_token);
     L->routes.pair_rank = reinterpret_cast<int32_t *>(b + w.pair_rank);
@@ -190,9 +190,6 @@ int finish_create(moe_ffn_layer *L) {
     if (const char *env = std::getenv("MOE_FFN_MFMA_ROUTES")) L->mfma_routes = std::atoi(env);
     if (const char *env = std::getenv("MOE_FFN_DECODE")) L->decode_mode = std::atoi(env) ? 1 : 0;
     if (const char *env = std::getenv("MOE_FFN_STREAMS")) L->two_streams = std::atoi(env) != 1;
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, L->device) == hipSuccess && cus > 0)
-        L->cu_count = cus;
     return hipDeviceSynchronize();
 }
 
@@ -380,16 +377,14 @@ moe::FfnArgs base_args(moe_ffn_layer *L, int tokens, int *error) {
     a.pairs_bound = static_cast<int>(pairs_capacity(L->shape, tokens));
     a.mfma_min = L->active_mfma_min;
     a.error = error;
-    a.cu_count = L->cu_count;
+    a.xhalf = L->xhalf;
     return a;
 }
 
 // The activation planes a batch fills: the fp16 operand plane only when some
 // of its groups can go to an MFMA kernel that reads it.
-Act activation_planes(const moe_ffn_layer *L, bool mfma) {
-    Act xq = L->xq;
-    if (!mfma || L->shape.H / 32 > moe::kHalfMaxBlocks) xq.half = nullptr;
-    return xq;
+moe::ActOut activation_planes(const moe_ffn_layer *L, bool mfma) {
+    return moe::ActOut{L->xq, mfma ? L->xhalf : nullptr};
 }
 
 }  // namespace
@@ -507,7 +502,7 @@ int run_stage(moe_ffn_layer *L, int stage, const float *x, const int32_t *ids, c
         if (stage == MOE_STAGE_DOWN) return moe::launch_decode_down_fold(d, s);
         return stage >= MOE_STAGE_PREPARE && stage <= MOE_STAGE_FOLD ? hipSuccess : kInvalid;
     }
-    const Act xq = activation_planes(L, L->active_mfma_min > 0);
+    const moe::ActOut xq = activation_planes(L, L->active_mfma_min > 0);
     switch (stage) {
     case MOE_STAGE_PREPARE:
         if (L->x_q8_in) {   // grouping only, then the given Q8 rows into the activation planes
@@ -661,7 +656,7 @@ int moe_ffn_group_routes(moe_ffn_layer *L, const int32_t *ids, const float *weig
         return kInvalid;
     const auto s = static_cast<hipStream_t>(stream);
     const Shape &sh = L->shape;
-    hipError_t r = moe::launch_prepare(nullptr, ids, weights, tokens, sh, L->xq, L->routes, 0, error, s);
+    hipError_t r = moe::launch_prepare(nullptr, ids, weights, tokens, sh, moe::ActOut{L->xq}, L->routes, 0, error, s);
     if (r != hipSuccess) return r;
     const size_t P = static_cast<size_t>(tokens) * sh.k;
     if ((r = hipMemcpyAsync(counts, L->routes.counts, sh.E * 4, hipMemcpyDeviceToDevice, s)) != hipSuccess) return r;
@@ -705,7 +700,7 @@ int moe_ffn_expert_down(moe_ffn_layer *L, int expert, const void *middle_q8, int
     if (mfma && !aligned(y, 16)) return kInvalid;   // the MFMA down kernel stores float4 rows
     const auto s = static_cast<hipStream_t>(stream);
     const Shape &sh = L->shape;
-    hipError_t r = moe::launch_canonical_to_planes(middle_q8, L->mq, columns * (sh.I / 32), s);
+    hipError_t r = moe::launch_canonical_to_planes(middle_q8, moe::ActOut{L->mq}, columns * (sh.I / 32), s);
     if (r != hipSuccess) return r;
     if ((r = moe::launch_single_expert_items(sh, L->routes, expert, columns, mfma, s)) != hipSuccess) return r;
     moe::FfnArgs a = base_args(L, columns, error);
@@ -809,7 +804,7 @@ int moe_ffn_debug_last(moe_ffn_layer *L, void *x_q8, void *middle_q8, int32_t *r
     if (L->last_decode) {
         // The decode path does not group: group the same routes now (the last
         // inputs must still be valid) and reorder its middle rows to match.
-        if ((r = moe::launch_prepare(nullptr, L->last_ids, L->last_weights, N, sh, L->xq, L->routes, L->active_mfma_min,
+        if ((r = moe::launch_prepare(nullptr, L->last_ids, L->last_weights, N, sh, moe::ActOut{L->xq}, L->routes, L->active_mfma_min,
                                      L->diag_error, s)) != hipSuccess)
             return r;
         if (middle_q8 && (r = moe::launch_decode_middle_grouped(L->mq, L->routes, sh, N, middle_q8, s)) != hipSuccess)
@@ -838,7 +833,7 @@ int moe_ffn_last_stats(moe_ffn_layer *L, int32_t *stream_items, int32_t *mfma_it
     if (hipStreamSynchronize(s) != hipSuccess) return kInvalid;
     if (L->last_decode && L->last_tokens > 0) {   // group the last batch's routes (not done by the decode path)
         const hipError_t g = moe::launch_prepare(nullptr, L->last_ids, L->last_weights, L->last_tokens, L->shape,
-                                                 L->xq, L->routes, L->active_mfma_min, L->diag_error, s);
+                                                 moe::ActOut{L->xq}, L->routes, L->active_mfma_min, L->diag_error, s);
         if (g != hipSuccess) return g;
     }
     hipError_t r = hipMemcpyAsync(c, L->routes.item_counts, sizeof(c), hipMemcpyDeviceToHost, s);

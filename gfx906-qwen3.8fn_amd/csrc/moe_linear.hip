@@ -527,15 +527,15 @@ bool use_half(const moe_linear *L, int columns) {
 
 // Planes for `columns` columns at `base_ptr`: fp16 operands (half) or codes,
 // then heads.
-moe::Act staging_planes(const moe_linear *L, void *base_ptr, int columns, bool half) {
+moe::ActOut staging_planes(const moe_linear *L, void *base_ptr, int columns, bool half) {
     auto *base = static_cast<uint8_t *>(base_ptr);
     const size_t blocks = static_cast<size_t>(columns) * L->nb;
-    if (half) return moe::Act{nullptr, reinterpret_cast<uint32_t *>(base + blocks * 64), reinterpret_cast<uint16_t *>(base)};
-    return moe::Act{base, reinterpret_cast<uint32_t *>(base + blocks * 32)};
+    if (half) return moe::ActOut{{nullptr, reinterpret_cast<uint32_t *>(base + blocks * 64)}, reinterpret_cast<uint16_t *>(base)};
+    return moe::ActOut{{base, reinterpret_cast<uint32_t *>(base + blocks * 32)}};
 }
 
 // x_q8: canonical Q8_1 columns read in place, else the planes xq.
-int launch_mfma(const moe_linear *L, moe::Act xq, const void *x_q8, int columns, float *y, hipStream_t s) {
+int launch_mfma(const moe_linear *L, moe::ActOut xq, const void *x_q8, int columns, float *y, hipStream_t s) {
     moe::LinearMfmaArgs a{};
     a.codes = L->codes;
     a.scales = L->scales;
@@ -672,7 +672,7 @@ int moe_linear_forward_q8(moe_linear *L, const void *x_q8, int columns, float *y
     const auto s = static_cast<hipStream_t>(stream);
     // The MFMA kernel reads the canonical blocks in place: no staging, so
     // any column count qualifies.
-    if (use_mfma_within(L, columns, 65536)) return launch_mfma(L, moe::Act{}, x_q8, columns, y, s);
+    if (use_mfma_within(L, columns, 65536)) return launch_mfma(L, moe::ActOut{}, x_q8, columns, y, s);
     return launch_vector(L, x_q8, columns, y, s);
 }
 
@@ -681,7 +681,7 @@ int moe_linear_apply(moe_linear *L, const float *x, int columns, float *y, int *
         return kInvalid;
     const auto s = static_cast<hipStream_t>(stream);
     if (use_mfma(L, columns)) {
-        const moe::Act xq = staging_planes(L, L->q8, columns, use_half(L, columns));
+        const moe::ActOut xq = staging_planes(L, L->q8, columns, use_half(L, columns));
         const hipError_t r = moe::launch_quantize_planes(x, xq, L->input, columns, error, s);
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
@@ -708,7 +708,7 @@ int moe_linear_apply_noalloc(moe_linear *L, const float *x, int columns, float *
     const auto s = static_cast<hipStream_t>(stream);
     const bool mfma = use_mfma_within(L, columns, 65536), half = mfma && use_half(L, columns);
     if (mfma && static_cast<size_t>(columns) * L->nb * (half ? kHalfPlaneBytes : 36) <= kNoallocScratchBytes) {
-        const moe::Act xq = staging_planes(L, ws, columns, half);
+        const moe::ActOut xq = staging_planes(L, ws, columns, half);
         const hipError_t r = moe::launch_quantize_planes(x, xq, L->input, columns, error, s);
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
@@ -718,7 +718,7 @@ int moe_linear_apply_noalloc(moe_linear *L, const float *x, int columns, float *
     if (r != hipSuccess) return r;
     // Batches whose operand planes outgrow the array: canonical blocks, which
     // the MFMA kernels read as well.
-    if (mfma) return launch_mfma(L, moe::Act{}, ws, columns, y, s);
+    if (mfma) return launch_mfma(L, moe::ActOut{}, ws, columns, y, s);
     return launch_vector(L, ws, columns, y, s);
 }
 
