@@ -301,10 +301,11 @@ __global__ __launch_bounds__(kHtThreads, Dbg ? 2 : 3) void k_gate_up_half(FfnArg
                         static_cast<int>((F0[v] + F1[v]) * kHalfScale);
         }
     });
-    // The park areas are free (the tree's last barrier): both waves' sums.
-    float (*xch)[16][64] = reinterpret_cast<float (*)[16][64]>(&st.park[2 * rs][0]);   // [mat]
+    // Both waves' sums, each in its own wave's park area: no barrier follows the
+    // merges of nodes without blocks, so the other wave may still be merging.
+    const float (*xch[2])[64] = {st.park[2 * rs][0], st.park[2 * rs + 1][0]};   // [mat][v][lane]
 #pragma unroll
-    for (int v = 0; v < 16; ++v) xch[mat][v][lane] = res[v];
+    for (int v = 0; v < 16; ++v) st.park[wave][0][v][lane] = res[v];
     __syncthreads();
     if (!active) return;
     // Wave `mat` finishes tokens 16 mat .. + 15: lane l rows 8 (l / 16) .. + 7 of
