@@ -252,10 +252,8 @@ __device__ __forceinline__ void half_tree(HalfLds &st, const HalfTile &t, int wa
 }
 
 // Gate / up: waves 2r and 2r + 1 take the gate and up rows of row tile r (two
-// tiles of 32 rows a workgroup) against token tile `sub` of an MFMA item; the
-// two waves then share the SiLU, the quantisation and the stores, 16 tokens
-// each (the IEEE divisions and expf of one wave for 32 tokens cost as much as
-// 4.5 % of the main loop's instructions).
+// tiles of 32 rows a workgroup) against token tile `sub` of an MFMA item, then
+// share the tile's SiLU and quantisation (finish_gate_up).
 constexpr int kGuTiles = kHtWaves / 2;
 
 template<bool Full, bool Dbg>
@@ -308,34 +306,7 @@ __global__ __launch_bounds__(kHtThreads, Dbg ? 2 : 3) void k_gate_up_half(FfnArg
     for (int v = 0; v < 16; ++v) st.park[wave][0][v][lane] = res[v];
     __syncthreads();
     if (!active) return;
-    // Wave `mat` finishes tokens 16 mat .. + 15: lane l rows 8 (l / 16) .. + 7 of
-    // token 16 mat + l % 16.
-    const int part = lane >> 4, m = 16 * mat + (lane & 15), j = kSub * sub + m;
-    int flags = 0;
-    float mid[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int v = 8 * (part & 1) + e, l = 32 * (part >> 1) + m;
-        mid[e] = silu_mul(xch[0][v][l], xch[1][v][l], flags);
-    }
-    float keep[8];
-    if constexpr (Dbg) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) keep[e] = mid[e];
-    }
-    const Q8Part<4> q8 = quantize_part<4>(mid);
-    if (j < ncols) {
-        const size_t pair = static_cast<size_t>(first + j), mb = pair * nbi + R0 / 32;
-        *reinterpret_cast<uint2 *>(a.mq.codes + mb * 32 + 8 * part) = make_uint2(q8.codes[0], q8.codes[1]);
-        if (part == 0) a.mq.heads[mb] = q8.head;
-        if constexpr (Dbg) {
-            if (a.middle_f32)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) a.middle_f32[pair * I + R0 + 8 * part + e] = keep[e];
-        }
-        const int f = flags | (part == 0 ? q8.flags : 0);
-        if (f) atomicOr(a.error, f);
-    }
+    finish_gate_up<Dbg>(a, xch[0], xch[1], mat, first, kSub * sub, ncols, R0);
 }
 
 // Q4_0 linear on wide grids: 4 row tiles of 32 a workgroup against the same 32

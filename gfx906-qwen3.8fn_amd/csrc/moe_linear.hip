@@ -24,10 +24,11 @@
 // lane's 8 row codes are eight 16-byte loads and its 8 scales one more.
 //
 // Wide batches (at least 32 columns and kMfmaMinOutputs outputs) go to
-// int8 MFMA instead (k_linear_mfma in moe_mfma.hip): the same fp32 order, with
-// the per-fragment integer dots from v_mfma_i32_32x32x16_i8.  forward_q8's
-// MFMA launch reads the caller's canonical blocks in place (any column
-// count); apply quantizes into split planes in the handle's workspace.
+// MFMA instead: the same fp32 order, with the per-fragment integer dots from
+// v_mfma_i32_32x32x16_i8 (k_linear_mfma in moe_leaf.hpp) or, on the widest
+// Q4_0 grids, from fp16 operands (k_linear_half in moe_half.hpp).
+// forward_q8's MFMA launch reads the caller's canonical blocks in place (any
+// column count); apply quantizes into planes in the handle's workspace.
 //
 // Work: one wave per (8 rows, column tile).  The wave loads its 8 rows'
 // blocks once per 4 columns (2 when a row has more than 64 blocks) and keeps

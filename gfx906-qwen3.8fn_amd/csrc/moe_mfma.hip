@@ -1,4 +1,6 @@
-// Int8-MFMA grouped expert projections for prefill-width groups (gfx950).
+// Int8-MFMA grouped expert projections for prefill-width groups (gfx950): the
+// down projection, and gate / up of rows of more than 64 blocks (shorter rows:
+// moe_half.hpp).
 //
 // Replaces the reference's MMQ path (src/hip/mmq.hip:139-381, mmq<Q4_0,J>) and
 // the Session's MMVQ expert projections for wide groups
@@ -256,11 +258,9 @@ __device__ __forceinline__ void tile_dispatch(const TileArgs &t, int nsub, float
 // blocks) and kFoldGrouped (64).
 template<int Fold, bool Dbg>
 __global__ __launch_bounds__(128, 2) void k_gate_up_mfma(FfnArgs a) {
-    // Pending tree levels 3-4 per wave; after the tree the up wave's area
-    // carries its result to the gate wave.
+    // Pending tree levels 3-4 per wave; after the tree, the waves' results.
     __shared__ float park[2][2][16][64];
     __shared__ uint4 d4_lds[2][Fold == kFoldGrouped96 ? kGu96MaxBlocks : 1][4];   // [mat][block][32 halfs]
-    float (*xch)[64] = park[1][0];
     const int mat = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int H = a.shape.H, I = a.shape.I, nb = H / 32, nbi = I / 32;
     const int slices = nbi * kSubs;
@@ -317,35 +317,12 @@ __global__ __launch_bounds__(128, 2) void k_gate_up_mfma(FfnArgs a) {
     } else {
         fold_tree_multi<Dbg>(t, park[mat], lane, res);
     }
-    if (mat == 1) {
+    // Both waves' sums meet in LDS (each wave's own park area) and each wave
+    // finishes 16 tokens (finish_gate_up).
 #pragma unroll
-        for (int v = 0; v < 16; ++v) xch[v][lane] = res[v];
-    }
-    __syncthreads();   // (the up wave's tree is done with park[1]; the gate wave's with park[0])
-    if (mat != 0) return;
-    int flags = 0;
-    float mid[16];
-#pragma unroll
-    for (int v = 0; v < 16; ++v) mid[v] = silu_mul(res[v], xch[v][lane], flags);
-    float keep[16];
-    if constexpr (Dbg) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) keep[v] = mid[v];
-    }
-    const Q8Part<2> q8 = quantize_part<2>(mid);
-    if (j < ncols) {
-        const size_t mb = static_cast<size_t>(pair) * nbi + R0 / 32;
-        *reinterpret_cast<uint4 *>(a.mq.codes + mb * 32 + 16 * h) =
-            make_uint4(q8.codes[0], q8.codes[1], q8.codes[2], q8.codes[3]);
-        if (h == 0) a.mq.heads[mb] = q8.head;
-        if constexpr (Dbg) {
-            if (a.middle_f32)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) a.middle_f32[static_cast<size_t>(pair) * I + R0 + 16 * h + v] = keep[v];
-        }
-        const int f = flags | (h == 0 ? q8.flags : 0);
-        if (f) atomicOr(a.error, f);
-    }
+    for (int v = 0; v < 16; ++v) park[mat][0][v][lane] = res[v];
+    __syncthreads();
+    finish_gate_up<Dbg>(a, park[0][0], park[1][0], mat, first, kSub * sub, ncols, R0);
 }
 
 // ------------------------------------------------------------------ down ---
