@@ -145,7 +145,7 @@ int moe_ffn_group_routes(moe_ffn_layer *layer, const int32_t *ids, const float *
                          int32_t *route_rank, int *error, void *stream);
 
 /* Kernel path selection for the single-expert stages below: MFMA = the
- * int8-MFMA kernels of the grouped forward (AUTO selects them); STREAM = the
+ * MFMA kernels of the grouped forward (AUTO selects them); STREAM = the
  * per-token streaming-dot kernels. */
 enum { MOE_PATH_AUTO = 0, MOE_PATH_STREAM = 1, MOE_PATH_MFMA = 2 };
 
