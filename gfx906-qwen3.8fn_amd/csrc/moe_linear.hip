@@ -175,7 +175,7 @@ __global__ __launch_bounds__(64, ROWS == 4 ? (G == 4 ? 3 : 4) : 2) void k_linear
 // The vector kernel from fp32 columns, for the few columns of a decode step:
 // a workgroup of 4 waves quantizes all G columns into LDS itself (4 lanes a
 // block, the bytes of k_quantize) while its first weights are in flight, then
-// each wave takes 4 rows as k_linear does.  Bound by latency: a launch of its
+// each wave takes 4 rows as k_linear does.  x and a.y must not overlap.  Bound by latency: a launch of its
 // own for the quantisation costs about 2 us, repeating it in every workgroup
 // about 1.1 us per 64 blocks (2048 x 2048 at one column 4.93 -> 3.32 us).
 template<bool Q41, int G>
@@ -397,7 +397,13 @@ int block_bytes(int type) { return type == MOE_TYPE_Q4_1 ? 20 : 18; }
 // 2048 rows 4.81 / 4.49, 512 4.39 / 4.43, 8192 6.68 / 7.09; 256 blocks, 8192 x
 // 8192 at one 11.3 / 13.5.
 constexpr int kFusedBlocks = 80;
-bool use_fused(const moe_linear *L, int columns) {
+// Every workgroup of k_linear_fp32 reads all of x while others store y, so a
+// call whose x and y overlap (an in-place projection) keeps the two launches,
+// whose second one reads only the workspace.
+bool use_fused(const moe_linear *L, const float *x, int columns, const float *y) {
+    const auto x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+    const size_t x_bytes = static_cast<size_t>(columns) * L->input * 4, y_bytes = static_cast<size_t>(columns) * L->output * 4;
+    if (x0 < y0 + y_bytes && y0 < x0 + x_bytes) return false;
     return columns <= 4 && columns * L->nb <= kFusedBlocks && L->vector_g == 0 && L->vector_rows == 0;
 }
 
@@ -687,7 +693,7 @@ int moe_linear_apply(moe_linear *L, const float *x, int columns, float *y, int *
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
     }
-    if (use_fused(L, columns)) return launch_fused(L, x, columns, y, error, s);
+    if (use_fused(L, x, columns, y)) return launch_fused(L, x, columns, y, error, s);
     const hipError_t r = moe::launch_quantize_canonical(x, L->q8, L->input, columns, error, s);
     if (r != hipSuccess) return r;
     return moe_linear_forward_q8(L, L->q8, columns, y, stream);
@@ -714,7 +720,7 @@ int moe_linear_apply_noalloc(moe_linear *L, const float *x, int columns, float *
         if (r != hipSuccess) return r;
         return launch_mfma(L, xq, nullptr, columns, y, s);
     }
-    if (use_fused(L, columns)) return launch_fused(L, x, columns, y, error, s);
+    if (use_fused(L, x, columns, y)) return launch_fused(L, x, columns, y, error, s);
     const hipError_t r = moe::launch_quantize_canonical(x, ws, L->input, columns, error, s);
     if (r != hipSuccess) return r;
     // Batches whose operand planes outgrow the array: canonical blocks, which

@@ -308,14 +308,17 @@ int moe_linear_bytes(const moe_linear *linear, size_t *weight_bytes);
 int moe_linear_forward_q8(moe_linear *linear, const void *x_q8, int columns, float *y, void *stream);
 
 /* Matrix::apply for Q4 types (src/session.hip:561-591): fp32 x
- * [columns][input] is quantized to Q8_1 into the handle's workspace
- * (launch_quantize_q8_1 semantics; flags OR-ed into `error`), then
- * forward_q8.  columns 1..max_columns.  Calls on one handle must not
- * overlap (they share the workspace). */
+ * [columns][input] is quantized to Q8_1 (launch_quantize_q8_1 semantics;
+ * flags OR-ed into `error`), then forward_q8, with the same outputs whether
+ * the quantised columns pass through the handle's workspace or, for a few
+ * columns, stay inside the product's kernel.  columns 1..max_columns.  x and
+ * y may overlap (y == x for a square matrix): all of x is read before any of
+ * y is written.  Calls on one handle must not overlap (they share the
+ * workspace). */
 int moe_linear_apply(moe_linear *linear, const float *x, int columns, float *y, int *error, void *stream);
 
-/* moe_linear_apply without the handle's workspace: the Q8_1 staging of x
- * lives in a static device array of the library, 4 MiB per GPU (held until
+/* moe_linear_apply (x and y may overlap here as well) without the handle's
+ * workspace: the Q8_1 staging of x lives in a static device array of the library, 4 MiB per GPU (held until
  * the process ends), so this call allocates nothing and works on handles
  * created with max_columns = 0.  No counterpart in the reference: it is for
  * callers that cannot allocate (code under HIP graph capture, tight serving
