@@ -19,7 +19,7 @@ hipError_t launch_gate_up_half(const FfnArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_linear_half(const LinearMfmaArgs &a, hipStream_t s) {
-    if (a.nb > kHalfMaxBlocks || a.mins || !(a.q8 || (a.xq.half && a.xq.heads))) return hipErrorInvalidValue;
+    if (a.nb > kHalfMaxBlocks || !(a.q8 || (a.xq.codes && a.xq.heads))) return hipErrorInvalidValue;
     const unsigned groups = static_cast<unsigned>((a.row_tiles + kHtWaves - 1) / kHtWaves);
     const unsigned grid = (groups + 7u) / 8u * 8u * static_cast<unsigned>(a.col_tiles);
     if (a.nb == kGuMaxBlocks) return launch_linear_half_full(a, grid, s);

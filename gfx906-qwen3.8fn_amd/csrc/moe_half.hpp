@@ -332,7 +332,7 @@ __global__ __launch_bounds__(kHtThreads, 3) void k_linear_half(LinearMfmaArgs a)
     t.wr = buffer_rsrc(a.codes + static_cast<size_t>(R0) * row_bytes, 32u * row_bytes);
     t.sr = buffer_rsrc(a.scales + static_cast<size_t>(R0) * nb, 32u * static_cast<uint32_t>(nb) * 2u);
     const uint32_t blocks = static_cast<uint32_t>(a.N) * static_cast<uint32_t>(nb);
-    t.xr = Canon ? buffer_rsrc(a.q8, blocks * 36u) : buffer_rsrc(a.xq.half, blocks * 64u);
+    t.xr = Canon ? buffer_rsrc(a.q8, blocks * 36u) : buffer_rsrc(a.xq.codes, blocks * 64u);
     t.hr = Canon ? t.xr : buffer_rsrc(a.xq.heads, blocks * 4u);
     t.x_base = column_row(tid >> 3) * HtXStride<Canon>;
     t.h_base = column_row(tid & 31) * HtHStride<Canon>;

@@ -205,27 +205,31 @@ hipError_t launch_down_mfma(const FfnArgs &a, hipStream_t s);
 hipError_t launch_gate_up_half(const FfnArgs &a, hipStream_t s);
 hipError_t launch_gate_up_half_full(const FfnArgs &a, unsigned grid, hipStream_t s);
 
-// One Q4_0 matrix (planes, rows padded to a multiple of 32) against N
-// Q8_1 columns, in the reference MMVQ fp32 order, on MFMA (moe_mfma.hip);
-// used by moe_linear for wide column counts.
+// One matrix (planes, rows padded to a multiple of 32) against N Q8_1 columns,
+// in the reference MMVQ fp32 order, on MFMA; used by moe_linear for wide column
+// counts.  The Q4_0 kernels' arguments hold what they read and no more: 16
+// bytes of unused pointers cost them 0.05 us a launch (2048 x 2048 at 48 / 96
+// columns, graph replay, 8.15 / 8.73 -> 8.11 / 8.68 us).
 struct LinearMfmaArgs {
     const uint8_t *codes;     // [Mp][nb][16 B]
     const uint16_t *scales;   // [Mp/8][nb][8]
-    const uint16_t *mins;     // Q4_1: same order as scales; Q4_0: null
-    ActOut xq;                // [N][nb] planes, read when q8 is null: heads and codes, or (launch_linear_half) half
+    Act xq;                   // [N][nb] planes, read when q8 is null; launch_linear_half: codes is the fp16 operand plane
     const uint8_t *q8;        // canonical Q8_1 columns [N][nb][36 B] {d, s, qs[32]}, or null
     float *y;                 // [N][M]
     int nb, M, N;
     int row_tiles;            // Mp / 32
     int col_tiles;            // ceil(N / 32)
-    int waves;                // waves per workgroup: 4, or 8 (two tree nodes a wave)
+    int waves;                // Q4_0, waves per workgroup: 4, or 8 (two tree nodes a wave)
 };
-hipError_t launch_linear_mfma(const LinearMfmaArgs &a, hipStream_t s);
-// Q4_0 rows of at most 64 blocks on wide grids, on fp16 operands: xq.half or
-// canonical blocks (moe_half.hip, moe_half_full.hip).
+struct LinearMfmaQ41Args : LinearMfmaArgs {
+    const uint16_t *mins;     // same order as scales
+};
+hipError_t launch_linear_mfma(const LinearMfmaArgs &a, hipStream_t s);          // Q4_0 (moe_mfma.hip)
+hipError_t launch_linear_mfma_q41(const LinearMfmaQ41Args &a, hipStream_t s);   // Q4_1 (moe_linear_q41.hip)
+// Q4_0 rows of at most 64 blocks on wide grids, on fp16 operands: their plane
+// or canonical blocks (moe_half.hip, moe_half_full.hip).
 hipError_t launch_linear_half(const LinearMfmaArgs &a, hipStream_t s);
 hipError_t launch_linear_half_full(const LinearMfmaArgs &a, unsigned grid, hipStream_t s);
-hipError_t launch_linear_mfma_q41(const LinearMfmaArgs &a, unsigned grid, hipStream_t s);   // moe_linear_q41.hip
 
 hipError_t launch_fold(const float *contributions, size_t token_stride, const float *weights, int k,
                        const int32_t *pos_of, const float *shared, size_t shared_stride,

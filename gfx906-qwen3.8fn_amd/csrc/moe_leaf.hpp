@@ -5,6 +5,8 @@
 
 #include "moe_mfma_device.hpp"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace moe {
@@ -333,39 +335,56 @@ __device__ __forceinline__ v16i extra_dots(const ExtraBlk &E, int i, int shift) 
     return frag_mfma<F, Q41>(Blk{E.w[i], E.x[i]}, shift);
 }
 
+// The MFMA operands and scales of leaf kp's blocks kp (a) and kp + 32 (b).
+template<bool Q41> struct LeafOps {
+    uint32_t a[4], b[4];
+    BlkScale<Q41> sa, sb;
+    __device__ __forceinline__ LeafOps(const GuStage &g, const HalfGroup &G, int i, int kp, int h) {
+        const uint4 wi = G.w[i];
+        const uint32_t wv[4] = {wi.x, wi.y, wi.z, wi.w};
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const auto r = __builtin_amdgcn_permlane32_swap(nibbles<Q41>(wv[d], 0), nibbles<Q41>(wv[d], 4), false, false);
+            a[d] = r[0];   // block kp: low nibbles (lanes < 32), high nibbles (lanes >= 32)
+            b[d] = r[1];   // block kp + 32
+        }
+        sa = staged_scale<Q41>(g, kp, h, i ? G.ha.y : G.ha.x);
+        sb = staged_scale<Q41>(g, kp + 32, h, i ? G.hb.y : G.hb.x);
+    }
+};
+
 // Leaf kp with block kp + 64 in chain A: v = (A0 + B0) + (A1 + B1), with
 // A_f = fma(d4', t', fma(d4, t, +0)) over blocks kp, kp + 64 and B_f block
 // kp + 32's value, as leaf_grouped without the extra block.
 template<bool Dbg, bool Q41>
 __device__ __forceinline__ void leaf_grouped_extra(const GuTile &t, const GuStage &g, const HalfGroup &G,
-                                                   const ExtraBlk &E, int i, int kp, int h, const uint32_t (&opa)[4],
-                                                   const uint32_t (&opb)[4], const BlkScale<Q41> &sa,
-                                                   const BlkScale<Q41> &sb, float (&v)[16]) {
+                                                   const ExtraBlk &E, int i, int kp, int h, const LeafOps<Q41> &o,
+                                                   float (&v)[16]) {
     const uint4 xa = G.xa[i], xb = G.xb[i];
     float u0[16];
     v16i keep_a0, keep_b0, keep_e0;
     {
         float za[16];
-        const v16i Ia = frag_mfma2(opa[0], opa[1], xa.x, xa.y);
+        const v16i Ia = frag_mfma2(o.a[0], o.a[1], xa.x, xa.y);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) za[j] = frag_value<Q41>(Ia[j], sa, j);
+        for (int j = 0; j < 16; ++j) za[j] = frag_value<Q41>(Ia[j], o.sa, j);
         const v16i Ie = extra_dots<0, Q41>(E, i, t.shift);
         fragment_scale<Q41>(za, Ie, staged_scale<Q41>(g, kp + 64, h, E.hd[i]));
-        const v16i Ib = frag_mfma2(opb[0], opb[1], xb.x, xb.y);
+        const v16i Ib = frag_mfma2(o.b[0], o.b[1], xb.x, xb.y);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) u0[j] = za[j] + frag_value<Q41>(Ib[j], sb, j);
+        for (int j = 0; j < 16; ++j) u0[j] = za[j] + frag_value<Q41>(Ib[j], o.sb, j);
         if constexpr (Dbg) { keep_a0 = Ia; keep_b0 = Ib; keep_e0 = Ie; }
     }
     {
         float za[16];
-        const v16i Ia = frag_mfma2(opa[2], opa[3], xa.z, xa.w);
+        const v16i Ia = frag_mfma2(o.a[2], o.a[3], xa.z, xa.w);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) za[j] = frag_value<Q41>(Ia[j], sa, j);
+        for (int j = 0; j < 16; ++j) za[j] = frag_value<Q41>(Ia[j], o.sa, j);
         const v16i Ie = extra_dots<1, Q41>(E, i, t.shift);
         fragment_scale<Q41>(za, Ie, staged_scale<Q41>(g, kp + 64, h, E.hd[i]));
-        const v16i Ib = frag_mfma2(opb[2], opb[3], xb.z, xb.w);
+        const v16i Ib = frag_mfma2(o.b[2], o.b[3], xb.z, xb.w);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) v[j] = u0[j] + (za[j] + frag_value<Q41>(Ib[j], sb, j));
+        for (int j = 0; j < 16; ++j) v[j] = u0[j] + (za[j] + frag_value<Q41>(Ib[j], o.sb, j));
         if constexpr (Dbg) {
             store_dots<Dbg>(t, kp, keep_a0, Ia);
             store_dots<Dbg>(t, kp + 32, keep_b0, Ib);
@@ -375,23 +394,25 @@ __device__ __forceinline__ void leaf_grouped_extra(const GuTile &t, const GuStag
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template<bool Dbg, bool Extra, bool Q41>
+// Shared: with an extra block, the operands are formed once, before the uniform
+// branch; else on each side of it (the compiler then schedules the two sides
+// each on its own).  us, shared / not, rows of 80 blocks x 2560: planes at 200 /
+// 1,032 columns 28.2 / 86.2 against 28.7 / 87.0, Q4_1 91.1 against 91.8 at
+// 1,032; but canonical Q4_0 blocks 24.2 / 79.1 against 23.9 / 78.2, and the
+// gate / up kernel's layers lose 0.5 %.
+template<bool Dbg, bool Extra, bool Q41, bool Shared>
 __device__ __forceinline__ void leaf_grouped(const GuTile &t, const GuStage &g, const HalfGroup &G, int i, int kp, int h,
                                              float (&v)[16], const ExtraBlk &E) {
-    const uint4 wi = G.w[i];
-    const uint32_t wv[4] = {wi.x, wi.y, wi.z, wi.w};
-    uint32_t opa[4], opb[4];
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        const auto r = __builtin_amdgcn_permlane32_swap(nibbles<Q41>(wv[d], 0), nibbles<Q41>(wv[d], 4), false, false);
-        opa[d] = r[0];   // block kp: low nibbles (lanes < 32), high nibbles (lanes >= 32)
-        opb[d] = r[1];   // block kp + 32
-    }
-    const BlkScale<Q41> sa = staged_scale<Q41>(g, kp, h, i ? G.ha.y : G.ha.x);
-    const BlkScale<Q41> sb = staged_scale<Q41>(g, kp + 32, h, i ? G.hb.y : G.hb.x);
-    if constexpr (Extra) {
+    if constexpr (Extra && !Shared) {
         if (kp < t.nb - 64) {   // uniform
-            leaf_grouped_extra<Dbg, Q41>(t, g, G, E, i, kp, h, opa, opb, sa, sb, v);
+            leaf_grouped_extra<Dbg, Q41>(t, g, G, E, i, kp, h, LeafOps<Q41>(g, G, i, kp, h), v);
+            return;
+        }
+    }
+    const LeafOps<Q41> o(g, G, i, kp, h);
+    if constexpr (Extra && Shared) {
+        if (kp < t.nb - 64) {   // uniform
+            leaf_grouped_extra<Dbg, Q41>(t, g, G, E, i, kp, h, o, v);
             return;
         }
     }
@@ -399,15 +420,15 @@ __device__ __forceinline__ void leaf_grouped(const GuTile &t, const GuStage &g, 
     float u0[16];
     v16i keep_a0, keep_b0;
     {
-        const v16i Ia = frag_mfma2(opa[0], opa[1], xa.x, xa.y), Ib = frag_mfma2(opb[0], opb[1], xb.x, xb.y);
+        const v16i Ia = frag_mfma2(o.a[0], o.a[1], xa.x, xa.y), Ib = frag_mfma2(o.b[0], o.b[1], xb.x, xb.y);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) u0[j] = frag_value<Q41>(Ia[j], sa, j) + frag_value<Q41>(Ib[j], sb, j);
+        for (int j = 0; j < 16; ++j) u0[j] = frag_value<Q41>(Ia[j], o.sa, j) + frag_value<Q41>(Ib[j], o.sb, j);
         if constexpr (Dbg) { keep_a0 = Ia; keep_b0 = Ib; }
     }
     {
-        const v16i Ia = frag_mfma2(opa[2], opa[3], xa.z, xa.w), Ib = frag_mfma2(opb[2], opb[3], xb.z, xb.w);
+        const v16i Ia = frag_mfma2(o.a[2], o.a[3], xa.z, xa.w), Ib = frag_mfma2(o.b[2], o.b[3], xb.z, xb.w);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) v[j] = u0[j] + (frag_value<Q41>(Ia[j], sa, j) + frag_value<Q41>(Ib[j], sb, j));
+        for (int j = 0; j < 16; ++j) v[j] = u0[j] + (frag_value<Q41>(Ia[j], o.sa, j) + frag_value<Q41>(Ib[j], o.sb, j));
         if constexpr (Dbg) {
             store_dots<Dbg>(t, kp, keep_a0, Ia);
             store_dots<Dbg>(t, kp + 32, keep_b0, Ib);
@@ -470,8 +491,8 @@ __device__ __forceinline__ void fold_tree_grouped(const GuTile &t, const GuStage
         }
         half_load_w(t, w_off, p < 15 ? p + 1 : p, wn);   // node p + 1's weights in flight during node p
         float w[16], x[16];
-        leaf_grouped<Dbg, Extra, false>(t, g, G, 0, 2 * p, h, w, E);
-        leaf_grouped<Dbg, Extra, false>(t, g, G, 1, 2 * p + 1, h, x, E);
+        leaf_grouped<Dbg, Extra, false, false>(t, g, G, 0, 2 * p, h, w, E);
+        leaf_grouped<Dbg, Extra, false, false>(t, g, G, 1, 2 * p + 1, h, x, E);
 #pragma unroll
         for (int i = 0; i < 16; ++i) w[i] = w[i] + x[i];
         tree_merge(park, lane, p, w, l1, l2, res);
@@ -628,8 +649,8 @@ __device__ __forceinline__ void subtree(const GuTile &t, const GuStage &g, uint3
             }
             half_load_w(t, w_off, q < NPW - 1 ? p + 1 : p, wn);
             float w[16], x[16];
-            leaf_grouped<false, X, Q41>(t, g, G, 0, 2 * p, h, w, E);
-            leaf_grouped<false, X, Q41>(t, g, G, 1, 2 * p + 1, h, x, E);
+            leaf_grouped<false, X, Q41, Q41 || !Canon>(t, g, G, 0, 2 * p, h, w, E);
+            leaf_grouped<false, X, Q41, Q41 || !Canon>(t, g, G, 1, 2 * p + 1, h, x, E);
 #pragma unroll
             for (int i = 0; i < 16; ++i) w[i] = w[i] + x[i];
             if constexpr (NPW == 4) subtree4_merge(q, w, l1, l2, res);
@@ -655,6 +676,8 @@ __device__ __forceinline__ void subtree(const GuTile &t, const GuStage &g, uint3
     }
 }
 
+template<bool Q41> using LinearArgsOf = std::conditional_t<Q41, LinearMfmaQ41Args, LinearMfmaArgs>;
+
 // Canon: the columns are canonical Q8_1 blocks, read in place (codes at
 // byte 4 of each 36-byte block, the head at byte 0); else the split planes.
 // W = 8: eight waves of two level-1 nodes each, the roots combined
@@ -662,7 +685,7 @@ __device__ __forceinline__ void subtree(const GuTile &t, const GuStage &g, uint3
 // as the 4-wave form's (R0 + R1) + (R2 + R3) over 4-node subtrees -- for
 // launches whose 4-wave grid leaves SIMDs with one wave.
 template<int Fold, bool Canon, int W, bool Q41>
-__global__ __launch_bounds__(64 * W, W == 8 ? 1 : 2) void k_linear_mfma(LinearMfmaArgs a) {
+__global__ __launch_bounds__(64 * W, W == 8 ? 1 : 2) void k_linear_mfma(LinearArgsOf<Q41> a) {
     constexpr int NPW = 16 / W, VPW = 16 / W;   // level-1 nodes and finished values per wave
     __shared__ float roots[W][16][64];          // subtree roots [wave][value][lane]
     constexpr int SB = Fold == kFoldGrouped96 ? kGu96MaxBlocks : Fold == kFoldMulti ? 1 : kGuMaxBlocks;
@@ -681,7 +704,7 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 1 : 2) void k_linear_mfma(LinearMf
     GuTile t;
     t.wr = buffer_rsrc(a.codes + static_cast<size_t>(R0) * row_bytes, 32u * row_bytes);
     t.sr = buffer_rsrc(a.scales + static_cast<size_t>(R0) * nb, 32u * static_cast<uint32_t>(nb) * 2u);
-    t.mr = Q41 ? buffer_rsrc(a.mins + static_cast<size_t>(R0) * nb, 32u * static_cast<uint32_t>(nb) * 2u) : t.sr;
+    if constexpr (Q41) t.mr = buffer_rsrc(a.mins + static_cast<size_t>(R0) * nb, 32u * static_cast<uint32_t>(nb) * 2u);
     if constexpr (Canon) {
         t.xr = buffer_rsrc(a.q8, static_cast<uint32_t>(a.N) * static_cast<uint32_t>(nb) * 36u);
         t.hr = t.xr;
@@ -734,9 +757,9 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 1 : 2) void k_linear_mfma(LinearMf
         const float q0 = (roots[0][v][lane] + roots[1][v][lane]) + (roots[2][v][lane] + roots[3][v][lane]);
         if constexpr (W == 4) out[i] = q0;
         else out[i] = q0 + ((roots[4][v][lane] + roots[5][v][lane]) + (roots[6][v][lane] + roots[7][v][lane]));
-        // + 0: the reference's lanes start from +0, so none of its sums is -0
-        // (unused lanes are left out above).  Q4_1: half of the doubled sum.
-        out[i] = (Q41 ? 0.5f * out[i] : out[i]) + 0.0f;
+        // Q4_1: half of the doubled sum; + 0: the reference's lanes start from
+        // +0, so none of its sums is -0 (Q4_0's lane values do so as well).
+        if constexpr (Q41) out[i] = 0.5f * out[i] + 0.0f;
     }
     float *yr = a.y + static_cast<size_t>(c) * a.M + row;
     if constexpr (W == 4) {
@@ -751,8 +774,9 @@ __global__ __launch_bounds__(64 * W, W == 8 ? 1 : 2) void k_linear_mfma(LinearMf
 }
 
 template<bool Canon, int W, bool Q41>
-void launch_linear_mfma_t(const LinearMfmaArgs &a, unsigned grid, hipStream_t s) {
+void launch_linear_mfma_t(const LinearArgsOf<Q41> &a, hipStream_t s) {
     constexpr unsigned T = 64 * W;
+    const unsigned grid = static_cast<unsigned>((a.row_tiles + 7) / 8 * 8) * static_cast<unsigned>(a.col_tiles);
     // Only 64-block rows take the 8-wave form: for the other folds the
     // compiler's register allocator (with the iterative-ILP scheduler this
     // file is built with) fails on it.

@@ -543,11 +543,11 @@ moe::ActOut staging_planes(const moe_linear *L, void *base_ptr, int columns, boo
 
 // x_q8: canonical Q8_1 columns read in place, else the planes xq.
 int launch_mfma(const moe_linear *L, moe::ActOut xq, const void *x_q8, int columns, float *y, hipStream_t s) {
-    moe::LinearMfmaArgs a{};
+    moe::LinearMfmaQ41Args a{};
     a.codes = L->codes;
     a.scales = L->scales;
     a.mins = L->mins;
-    a.xq = xq;
+    a.xq = xq.half ? moe::Act{reinterpret_cast<uint8_t *>(xq.half), xq.heads} : moe::Act{xq};
     a.q8 = static_cast<const uint8_t *>(x_q8);
     a.y = y;
     a.nb = L->nb;
@@ -555,6 +555,7 @@ int launch_mfma(const moe_linear *L, moe::ActOut xq, const void *x_q8, int colum
     a.N = columns;
     a.row_tiles = L->Mp / 32;
     a.col_tiles = (columns + 31) / 32;
+    if (L->type == MOE_TYPE_Q4_1) return moe::launch_linear_mfma_q41(a, s);
     if (use_half(L, columns)) return moe::launch_linear_half(a, s);
     // 8-wave workgroups (two tree nodes a wave) for 64-block rows where the
     // 4-wave grid gives at most one workgroup per CU (us, 4 -> 8 waves,
@@ -562,7 +563,7 @@ int launch_mfma(const moe_linear *L, moe::ActOut xq, const void *x_q8, int colum
     // 10.5, 2048 x 512 at N = 320 / 512 10.2 / 10.9 -> 9.25 / 10.45, 2048 x
     // 1024 at N = 160 / 256 10.3 / 10.9 -> 9.35 / 10.5; larger grids lose:
     // 2048 x 2048 at N = 192 / 1032 16.0 / 54.5 -> 17.2 / 67.5).
-    a.waves = L->type == MOE_TYPE_Q4_0 && L->nb == 64 && static_cast<long>(a.row_tiles) * a.col_tiles <= 256 ? 8 : 4;
+    a.waves = L->nb == 64 && static_cast<long>(a.row_tiles) * a.col_tiles <= 256 ? 8 : 4;
     return moe::launch_linear_mfma(a, s);
 }
 

@@ -5,9 +5,9 @@
 
 namespace moe {
 
-hipError_t launch_linear_mfma_q41(const LinearMfmaArgs &a, unsigned grid, hipStream_t s) {
-    if (a.q8) launch_linear_mfma_t<true, 4, true>(a, grid, s);
-    else launch_linear_mfma_t<false, 4, true>(a, grid, s);
+hipError_t launch_linear_mfma_q41(const LinearMfmaQ41Args &a, hipStream_t s) {
+    if (a.q8) launch_linear_mfma_t<true, 4, true>(a, s);
+    else launch_linear_mfma_t<false, 4, true>(a, s);
     return hipGetLastError();
 }
 

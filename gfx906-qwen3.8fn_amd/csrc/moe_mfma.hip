@@ -970,15 +970,13 @@ unsigned mfma_grid(const FfnArgs &a, int slices) {
 }  // namespace
 
 hipError_t launch_linear_mfma(const LinearMfmaArgs &a, hipStream_t s) {
-    const unsigned grid = static_cast<unsigned>((a.row_tiles + 7) / 8 * 8) * static_cast<unsigned>(a.col_tiles);
     const bool w8 = a.waves == 8;
-    if (a.mins) return launch_linear_mfma_q41(a, grid, s);
     if (a.q8) {
-        if (w8) launch_linear_mfma_t<true, 8, false>(a, grid, s);
-        else launch_linear_mfma_t<true, 4, false>(a, grid, s);
+        if (w8) launch_linear_mfma_t<true, 8, false>(a, s);
+        else launch_linear_mfma_t<true, 4, false>(a, s);
     } else {
-        if (w8) launch_linear_mfma_t<false, 8, false>(a, grid, s);
-        else launch_linear_mfma_t<false, 4, false>(a, grid, s);
+        if (w8) launch_linear_mfma_t<false, 8, false>(a, s);
+        else launch_linear_mfma_t<false, 4, false>(a, s);
     }
     return hipGetLastError();
 }
