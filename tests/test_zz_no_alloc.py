@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import moe_ffn
+import oracle as O
 import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -89,3 +90,27 @@ def test_noalloc_without_workspace_and_limits():
     assert int(e.cpu()[0]) == 0 and bool((yb[:1820] == 0).all())
     lin0.close()
     ref.close()
+
+
+@pytest.mark.parametrize("qtype", [moe_ffn.TYPE_Q4_0, moe_ffn.TYPE_Q4_1])
+def test_noalloc_past_65536_columns(qtype):
+    """Rows of one block fit the static array up to 116,508 columns, past the
+    65,536 of the calls with a workspace; the MFMA kernels take them too."""
+    K, M, n, base = 32, 130, 116508, 256
+    rng = np.random.default_rng(qtype)
+    w = (W.q4_1_blocks(M, rng) if qtype == moe_ffn.TYPE_Q4_1 else W.q4_blocks(M, rng)).reshape(-1)
+    lin = moe_ffn.MoeLinear(qtype, K, M, w, max_columns=0)
+    x = W.activations(base, hidden=K, seed=9)
+    ref = (O.matrix_gpu_order_q41 if qtype == moe_ffn.TYPE_Q4_1 else O.matrix_gpu_order)(w, K, M, O.quantize_q8(x))
+    ref = torch.from_numpy(np.asarray(ref, np.float32).reshape(base, M)).to(DEV)
+    xd = torch.from_numpy(x).to(DEV).repeat(n // base + 1, 1)[:n].contiguous()
+    y = torch.empty((n, M), dtype=torch.float32, device=DEV)
+    e = torch.zeros(1, dtype=torch.int32, device=DEV)
+    lin.apply_noalloc(xd, y, e)
+    torch.cuda.synchronize()
+    want = ref.repeat(n // base + 1, 1)[:n]
+    assert torch.equal(y.view(torch.int32), want.view(torch.int32)) and int(e.cpu()[0]) == 0
+    big = torch.zeros((n + 1, K), dtype=torch.float32, device=DEV)
+    with pytest.raises(moe_ffn.MoeError):
+        lin.apply_noalloc(big, torch.empty((n + 1, M), dtype=torch.float32, device=DEV), e)
+    lin.close()
