@@ -381,9 +381,24 @@ bool half_rows(const moe_linear *L) {
     return L->type == MOE_TYPE_Q4_0 && L->nb >= kHalfMinBlocks && L->nb <= moe::kHalfMaxBlocks;
 }
 
-// Bytes per block of apply's workspace: the largest staging its matrix can use.
+// MFMA for wide batches that fit the staging area (`capacity` columns).
+bool use_mfma_within(const moe_linear *L, int columns, int capacity) {
+    if (columns < kMfmaMinColumns || columns > capacity || L->mfma_mode == 0) return false;
+    const long least = L->type == MOE_TYPE_Q4_1 && L->nb > 96 ? kMfmaMinOutputsQ41Long : kMfmaMinOutputs;
+    return L->mfma_mode == 1 || static_cast<long>(L->output) * columns >= least;
+}
+bool use_mfma(const moe_linear *L, int columns) { return use_mfma_within(L, columns, L->max_columns); }
+
+// Grids of at least kHalfMinGroups workgroups take the fp16-operand kernel.
+bool use_half(const moe_linear *L, int columns) {
+    const long groups = static_cast<long>((L->Mp / 32 + 3) / 4) * ((columns + 31) / 32);
+    return half_rows(L) && groups >= kHalfMinGroups;
+}
+
+// Bytes per block of apply's workspace: the largest staging that a batch of
+// at most max_columns can take (both rules only grow with the columns).
 size_t workspace_block(const moe_linear *L) {
-    return half_rows(L) ? kHalfPlaneBytes : 36;
+    return use_mfma(L, L->max_columns) && use_half(L, L->max_columns) ? kHalfPlaneBytes : 36;
 }
 
 int block_bytes(int type) { return type == MOE_TYPE_Q4_1 ? 20 : 18; }
@@ -517,20 +532,6 @@ int moe_linear_bytes(const moe_linear *L, size_t *weight_bytes) {
 }
 
 namespace {
-
-// MFMA for wide batches that fit the staging area (`capacity` columns).
-bool use_mfma_within(const moe_linear *L, int columns, int capacity) {
-    if (columns < kMfmaMinColumns || columns > capacity || L->mfma_mode == 0) return false;
-    const long least = L->type == MOE_TYPE_Q4_1 && L->nb > 96 ? kMfmaMinOutputsQ41Long : kMfmaMinOutputs;
-    return L->mfma_mode == 1 || static_cast<long>(L->output) * columns >= least;
-}
-bool use_mfma(const moe_linear *L, int columns) { return use_mfma_within(L, columns, L->max_columns); }
-
-// Grids of at least kHalfMinGroups workgroups take the fp16-operand kernel.
-bool use_half(const moe_linear *L, int columns) {
-    const long groups = static_cast<long>((L->Mp / 32 + 3) / 4) * ((columns + 31) / 32);
-    return half_rows(L) && groups >= kHalfMinGroups;
-}
 
 // Planes for `columns` columns at `base_ptr`: fp16 operands (half) or codes,
 // then heads.

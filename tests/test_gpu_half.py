@@ -76,3 +76,24 @@ def test_linear_wide_grid_matches_vector(K, M, N, monkeypatch):
     assert torch.equal(y.view(torch.int32), ref) and int(e.cpu()[0]) == 0
     V.close()
     L.close()
+
+
+@pytest.mark.parametrize("M,N,block", [(512, 4096, 36), (512, 5568, 36), (512, 5569, 68)])
+def test_linear_workspace_bytes(M, N, block):
+    """apply's workspace holds fp16 operand planes only where max_columns can
+    reach the kernel that reads them (4 row groups x 175 column tiles do)."""
+    w = W.q4_blocks(M * 64, np.random.default_rng(M)).reshape(-1)
+
+    def taken(columns):
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        L = moe_ffn.MoeLinear(moe_ffn.TYPE_Q4_0, 2048, M, w, max_columns=columns)
+        torch.cuda.synchronize()
+        return before - torch.cuda.mem_get_info()[0], L
+    taken(0)[1].close()   # the first one loads code objects
+    whole, L = taken(N)
+    L.close()
+    # The weights (0.6 MB) and the workspace are an allocation each, rounded up
+    # to 2 MiB or served from a chunk that is there: within 4 MiB either way,
+    # where 36 and 68 bytes a block lie 8 MiB and more apart.
+    assert abs(whole - N * 64 * block) <= 4 << 20, (whole, N * 64 * block)
