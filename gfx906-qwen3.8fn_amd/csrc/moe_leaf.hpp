@@ -473,9 +473,10 @@ __device__ __forceinline__ void tree_merge(float (*park)[16][64], int lane, int 
     }
 }
 
-template<bool Dbg, bool Extra = false>
-__device__ __forceinline__ void fold_tree_grouped(const GuTile &t, const GuStage &g, uint32_t w_off, float (*park)[16][64],
-                                                  int lane, uint4 (&wn)[2], float (&res)[16]) {
+// The tree of a row of 65..96 blocks.
+template<bool Dbg>
+__device__ __forceinline__ void fold_tree_grouped96(const GuTile &t, const GuStage &g, uint32_t w_off, float (*park)[16][64],
+                                                    int lane, uint4 (&wn)[2], float (&res)[16]) {
     // wn: node 0's weight half, already in flight.
     const int h = lane >> 5;
     float l1[16], l2[16];
@@ -486,13 +487,11 @@ __device__ __forceinline__ void fold_tree_grouped(const GuTile &t, const GuStage
         G.w[1] = wn[1];
         half_load_x(t, p, G);
         ExtraBlk E;
-        if constexpr (Extra) {
-            if (2 * p < t.nb - 64) extra_load(t, p, E);   // uniform
-        }
+        if (2 * p < t.nb - 64) extra_load(t, p, E);   // uniform
         half_load_w(t, w_off, p < 15 ? p + 1 : p, wn);   // node p + 1's weights in flight during node p
         float w[16], x[16];
-        leaf_grouped<Dbg, Extra, false, false>(t, g, G, 0, 2 * p, h, w, E);
-        leaf_grouped<Dbg, Extra, false, false>(t, g, G, 1, 2 * p + 1, h, x, E);
+        leaf_grouped<Dbg, true, false, false>(t, g, G, 0, 2 * p, h, w, E);
+        leaf_grouped<Dbg, true, false, false>(t, g, G, 1, 2 * p + 1, h, x, E);
 #pragma unroll
         for (int i = 0; i < 16; ++i) w[i] = w[i] + x[i];
         tree_merge(park, lane, p, w, l1, l2, res);
@@ -553,33 +552,7 @@ __device__ __forceinline__ void fold_tree_multi(const GuTile &t, float (*park)[1
         fold_leaf_multi<Dbg, false, false>(t, 2 * p + 1, x);
 #pragma unroll
         for (int i = 0; i < 16; ++i) w[i] = w[i] + x[i];
-        if ((p & 1) == 0) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) l1[i] = w[i];
-            continue;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) w[i] = l1[i] + w[i];
-        if ((p & 2) == 0) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) l2[i] = w[i];
-            continue;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) w[i] = l2[i] + w[i];
-        int lvl = 0;
-        for (; lvl < 2; ++lvl) {
-            if (((p >> (lvl + 2)) & 1) == 0) break;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) w[i] = park[lvl][i][lane] + w[i];
-        }
-        if (lvl < 2) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) park[lvl][i][lane] = w[i];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) res[i] = w[i];
-        }
+        tree_merge(park, lane, p, w, l1, l2, res);
     }
 }
 

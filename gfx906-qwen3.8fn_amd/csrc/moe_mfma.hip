@@ -313,7 +313,7 @@ __global__ __launch_bounds__(128, 2) void k_gate_up_mfma(FfnArgs a) {
         }
         __syncthreads();
         const GuStage g{reinterpret_cast<const uint32_t *>(&d4_lds[mat][0][0]), nullptr};
-        fold_tree_grouped<Dbg, true>(t, g, w_off, park[mat], lane, wn, res);
+        fold_tree_grouped96<Dbg>(t, g, w_off, park[mat], lane, wn, res);
     } else {
         fold_tree_multi<Dbg>(t, park[mat], lane, res);
     }
