@@ -507,18 +507,21 @@ struct LaneExpfTable {
     }
 };
 
-// SiLU(g)*u with the reference's sanitisation (src/hip/linear.hip:106-120),
-// expf's table read through `table` (MoeExpfTable: memory; LaneExpfTable:
-// registers, the whole wave calling).
+// SiLU(g)*u with the reference's sanitisation (src/hip/linear.hip:106-120): a
+// nonfinite value makes its own element 0 and is OR-ed into flags (a caller's
+// other elements keep their values).  expf's table is read through `table`
+// (MoeExpfTable: memory; LaneExpfTable: registers, the whole wave calling).
 template<typename Table>
 __device__ __forceinline__ float silu_mul(float g, float u, int &flags, const Table &table) {
-    if (!isfinite(g)) { flags |= 1; g = 0.0f; }
-    if (!isfinite(u)) { flags |= 1; u = 0.0f; }
+    int f = 0;
+    if (!isfinite(g)) { f |= 1; g = 0.0f; }
+    if (!isfinite(u)) { f |= 1; u = 0.0f; }
     float a = g / (1.0f + moe_expf_with(-g, table));
-    if (!isfinite(a)) { flags |= 2; a = 0.0f; }
+    if (!isfinite(a)) { f |= 2; a = 0.0f; }
     float v = a * u;
-    if (!isfinite(v)) { flags |= 2; v = 0.0f; }
-    return flags ? 0.0f : v;
+    if (!isfinite(v)) { f |= 2; v = 0.0f; }
+    flags |= f;
+    return f ? 0.0f : v;
 }
 
 __device__ __forceinline__ float silu_mul(float g, float u, int &flags) {

@@ -54,6 +54,36 @@ def test_gate_up_tile_edges(H, I, columns):
     L.close()
 
 
+@pytest.mark.parametrize("H", [2048, 1984, 2560, 4096])   # the fp16 forms; int8 for 65..96 blocks and past 96
+def test_gate_up_nonfinite_rows(H):
+    """Rows whose gate or up is nonfinite make their own middle element 0 and
+    raise bit 1, as the reference's per-element sanitisation does; every other
+    row of the 32-row block keeps its value, on both kernel paths."""
+    I, columns, nb = 64, 40, H // 32
+    rows = {3: np.inf, 4: -np.inf, 17: np.nan, 33: np.inf}
+    clean = W.q4_bank(1, hidden=H, intermediate=I, seed=H).reshape(3, -1).copy()
+    dirty = clean.copy()
+    for r, v in rows.items():
+        blocks = [m.reshape(I, nb, 18) for m in (clean[0], clean[1])]
+        for b in blocks:
+            b[r, :, :2] = 0                       # a row of zero blocks: gate = up = 0
+        which = dirty[r & 1].reshape(I, nb, 18)   # gate (0) or up (1)
+        which[r, nb // 2, :2] = np.array([v], np.float16).view(np.uint8)
+    x = W.activations(columns, hidden=H, seed=H + 1)
+    xq = O.quantize_q8(x)
+    ref = O.expert_forward(clean[0], clean[1], clean[2], H, I, xq)
+    xd = torch.from_numpy(np.ascontiguousarray(xq).view(np.uint8).reshape(columns, -1)).to(DEV)
+    L = moe_ffn.MoeLayer(H, I, 1, 1, False, columns, experts_q4=dirty.reshape(-1))
+    for path in (moe_ffn.PATH_STREAM, moe_ffn.PATH_MFMA):
+        got = L.expert_gate_up(0, xd, columns, path=path)
+        torch.cuda.synchronize()
+        assert int(got["error"].cpu()[0]) == 1, path
+        assert np.array_equal(got["middle"].cpu().numpy().view(np.uint32), ref["middle"].view(np.uint32)), path
+        assert np.array_equal(got["middle_q8"].cpu().numpy().reshape(-1),
+                              np.ascontiguousarray(ref["middle_q8"]).view(np.uint8).reshape(-1)), path
+    L.close()
+
+
 @pytest.mark.parametrize("K,M,N", [(1024, 2820, 1000), (2048, 2820, 1000), (1984, 2816, 1001)])
 def test_linear_wide_grid_matches_vector(K, M, N, monkeypatch):
     """Grids wide enough for the fp16-operand linear (canonical input, planes,
