@@ -6,7 +6,7 @@ unchanged.  And, as the reference proves for its CPU jobs
 (tests/cpu_expert_test.cpp:25-55), the hot path allocates nothing: 100
 forwards leave the device's free memory (hipMemGetInfo) unchanged.
 
-Paths covered: quantize, device router, the decode path (8 tokens), grouped
+Paths covered: quantize (both kernels), device router, the decode path (8 tokens), grouped
 streaming (64 tokens), grouped MFMA + streaming (1024 tokens, Zipf 1.1), a
 Q4_1-down layer (decode and grouped), forward_q8, debug_last's middle rows,
 the combine, and the quantized linear (vector and MFMA kernels).
@@ -171,9 +171,35 @@ def test_quantize_router_combine_guards():
     assert int(err.cpu()[0]) == 0
 
 
+@pytest.mark.parametrize("cols,width", [(255, 2048), (256, 2048), (257, 2080), (33, 16384)])
+def test_quantize_around_its_size_rule(cols, width):
+    """The quantizer's two kernels below, at and above 524,288 elements, the
+    last workgroup partly filled (257 x 2080: one block of 64): the oracle's
+    bytes from a base that is only 4-byte aligned, poisoned first and last
+    blocks as zeros with bit 1 raised, and nothing stored around the output."""
+    nb = width // 32
+    x = W.activations(cols, hidden=width, seed=cols)
+    ref = np.ascontiguousarray(O.quantize_q8(x)).view(np.uint8).reshape(cols, nb, 36).copy()
+    A = Arena(16 << 20)
+    xs = A.take((cols * width + 1,), torch.float32, np.concatenate([[0.0], x.reshape(-1)]).astype(np.float32))[1:]
+    q = A.take((cols, nb * 36), torch.uint8)
+    err = A.take((1,), torch.int32, np.zeros(1, np.int32))
+    call = lambda: moe_ffn.library().moe_quantize_q8_1(moe_ffn._ptr(xs), moe_ffn._ptr(q), width, cols,  # noqa: E731
+                                                       moe_ffn._ptr(err), moe_ffn._stream(None))
+    assert call() == 0
+    A.check("quantize")
+    assert np.array_equal(q.cpu().numpy().reshape(cols, nb, 36), ref) and int(err.cpu()[0]) == 0
+    xs[5], xs[-3] = float("nan"), float("-inf")
+    ref[0, 0] = ref[-1, -1] = 0
+    assert call() == 0
+    A.check("quantize, poisoned")
+    assert np.array_equal(q.cpu().numpy().reshape(cols, nb, 36), ref) and int(err.cpu()[0]) == 1
+
+
 @pytest.mark.parametrize("K,M,N", [(2048, 2048, 1), (2048, 2048, 8), (2048, 2048, 256), (2560, 640, 33)])
 def test_linear_guards(K, M, N):
-    """Vector kernel (1, 8 and 33 columns) and MFMA kernel (256 columns)."""
+    """The vector kernel that quantizes (1 column), the vector kernel (8 and 33) and
+    the MFMA kernel (256)."""
     rng = np.random.default_rng(K + M + N)
     lin = moe_ffn.MoeLinear(moe_ffn.TYPE_Q4_0, K, M, W.q4_blocks(M * K // 32, rng).reshape(-1), max_columns=N)
     A = Arena(16 << 20)

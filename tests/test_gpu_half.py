@@ -1,7 +1,8 @@
 """GPU parity of the kernels on fp16 operands (csrc/moe_half.hpp) at the edges
 of their tiles: rows of 1..64 blocks (the 64-block form and the one that
 zero-fills missing blocks), an odd number of 32-row tiles (an idle second
-tile in the last workgroup), and token counts around the 32-token tiles.
+tile in the last workgroup), and token counts around the 32-token tiles; and
+of their inputs: codes of -128, nonfinite heads, rows and activations.
 Every comparison is bit for bit: the kernels keep the reference's fp32 order.
 """
 import numpy as np
@@ -84,7 +85,10 @@ def test_gate_up_nonfinite_rows(H):
     L.close()
 
 
-@pytest.mark.parametrize("K,M,N", [(1024, 2820, 1000), (2048, 2820, 1000), (1984, 2816, 1001)])
+@pytest.mark.parametrize("K,M,N", [
+    (1024, 2820, 1000), (2048, 2820, 1000), (1984, 2816, 1001),
+    (2048, 2819, 1001), (1056, 2821, 999),   # rows no multiple of 4: stored one value at a time
+])
 def test_linear_wide_grid_matches_vector(K, M, N, monkeypatch):
     """Grids wide enough for the fp16-operand linear (canonical input, planes,
     and both stagings of the no-allocation call) against the vector kernel,
@@ -127,3 +131,54 @@ def test_linear_workspace_bytes(M, N, block):
     # to 2 MiB or served from a chunk that is there: within 4 MiB either way,
     # where 36 and 68 bytes a block lie 8 MiB and more apart.
     assert abs(whole - N * 64 * block) <= 4 << 20, (whole, N * 64 * block)
+
+
+@pytest.mark.parametrize("K", [2048, 1056])
+def test_linear_canonical_extremes(K):
+    """Canonical blocks as a caller may hand them in: codes of -128, the largest
+    and smallest heads, and nonfinite ones, which reach their own column only.
+    Bit for bit the vector kernel's values; where those are NaN, NaN."""
+    M, N = 2820, 1000
+    rng = np.random.default_rng(K)
+    w = W.q4_blocks(M * K // 32, rng).reshape(-1)
+    q8 = rng.integers(-128, 128, (N, K // 32, 36), dtype=np.int64).astype(np.int8).view(np.uint8)
+    heads = rng.standard_normal((N, K // 32, 2)).astype(np.float16)
+    heads[1], heads[2], heads[3] = 65504.0, 2.0 ** -24, 0.0
+    for i, v in enumerate((np.inf, -np.inf, np.nan)):
+        heads[100 + i, K // 64, 0] = v
+        heads[110 + i, K // 32 - 1, 1] = v
+    q8[..., :4] = heads.view(np.uint8)
+    q8[4, :, 4:] = 0x80
+    q8[5, :, 4:] = 0x7f
+    q8[100:103, :, 4:12] = 0   # an infinite scale times a zero dot
+    x = torch.from_numpy(np.ascontiguousarray(q8).reshape(N, -1)).to(DEV)
+    L = moe_ffn.MoeLinear(moe_ffn.TYPE_Q4_0, K, M, w)
+    got = L.forward_q8(x, N)
+    # 8 columns at a time take the vector kernel.
+    ref = torch.cat([L.forward_q8(x[c:c + 8].contiguous(), 8) for c in range(0, N, 8)])
+    nan = torch.isnan(ref)
+    assert torch.equal(torch.isnan(got), nan)
+    assert bool(torch.isfinite(ref[:100]).all()) and not bool(torch.isfinite(ref[100:103]).any())
+    assert torch.equal(got[~nan].view(torch.int32), ref[~nan].view(torch.int32))
+    L.close()
+
+
+@pytest.mark.parametrize("H,I", [(2048, 512), (1984, 64), (2560, 640)])
+def test_grouped_layer_nonfinite_activations(H, I):
+    """A grouped batch whose groups go to MFMA: a block with a nonfinite value
+    counts as zeros and raises bit 1; a zeroed block gives the same outputs."""
+    E, N = 8, 300
+    L = moe_ffn.MoeLayer(H, I, E, 4, True, N, synthetic_seed=H)
+    x = W.activations(N, hidden=H, seed=H)
+    ids, w = W.routes_uniform(N, experts=E, k=4, seed=1)
+    zeroed = x.copy()
+    for t, e, v in ((0, 0, np.nan), (17, H - 1, np.inf), (N - 1, 40, -np.inf)):
+        x[t, e] = v
+        zeroed[t, e // 32 * 32:e // 32 * 32 + 32] = 0.0
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)  # noqa: E731
+    y, err = L.forward(dev(x), dev(ids), dev(w))
+    ref, ok = L.forward(dev(zeroed), dev(ids), dev(w))
+    assert int(err.cpu()[0]) == 1 and int(ok.cpu()[0]) == 0
+    assert L.last_stats()["mfma_items"] > 0
+    assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
+    L.close()

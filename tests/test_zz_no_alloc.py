@@ -46,7 +46,7 @@ def _run_pair(lin, n, seed):
     (2048, 2048, 256, 100, moe_ffn.TYPE_Q4_0),   # MFMA kernel, then MFMA again on fewer columns
     (2048, 2048, 96, 8, moe_ffn.TYPE_Q4_0),      # MFMA, then the vector kernel
     (2560, 640, 33, 3, moe_ffn.TYPE_Q4_0),       # vector kernel (rows of 80 blocks)
-    (640, 2560, 128, 1, moe_ffn.TYPE_Q4_1),      # Q4_1 (vector kernel only)
+    (640, 2560, 128, 1, moe_ffn.TYPE_Q4_1),      # Q4_1: MFMA, then the vector kernel that quantizes
 ])
 def test_noalloc_matches_apply_two_calls(K, M, first, second, qtype):
     rng = np.random.default_rng(K * 3 + M + first)
