@@ -560,8 +560,8 @@ enum { kFoldStaged = 0, kFoldGrouped = 1, kFoldMulti = 2, kFoldGrouped96 = 3 };
 
 
 // ---------------------------------------------------------------- linear ---
-// One Q4_0 matrix against wide column batches (moe_linear), in the gate/up
-// kernel's exact order without the SiLU epilogue.  The reference's pairwise
+// One matrix against wide column batches (moe_linear), in the gate/up kernel's
+// exact order (Q4_1: its own block value) without the SiLU epilogue.  The reference's pairwise
 // tree over the 16 level-1 nodes (leaves 2p, 2p+1; leaf k' = blocks k' and
 // k' + 32 and, past 64 blocks, their lane's later blocks) splits into four
 // 4-node subtrees whose roots combine as (R0 + R1) + (R2 + R3): workgroup =
@@ -587,7 +587,6 @@ __device__ __forceinline__ void subtree4_merge(int q, float (&w)[16], float (&l1
     for (int i = 0; i < 16; ++i) res[i] = l2[i] + w[i];
 }
 
-// wn: the wave's first node's weight half, already in flight (grouped folds).
 // The two-node form for 8-wave workgroups: res = node 0 + node 1.
 __device__ __forceinline__ void subtree2_merge(int q, float (&w)[16], float (&l1)[16], float (&res)[16]) {
     if ((q & 1) == 0) {
@@ -599,7 +598,8 @@ __device__ __forceinline__ void subtree2_merge(int q, float (&w)[16], float (&l1
     for (int i = 0; i < 16; ++i) res[i] = l1[i] + w[i];
 }
 
-// NPW level-1 nodes per wave (4: a 4-wave workgroup, 2: an 8-wave one).
+// NPW level-1 nodes per wave (4: a 4-wave workgroup, 2: an 8-wave one).  wn: the
+// wave's first node's weight half, already in flight (grouped folds).
 template<int Fold, bool Canon, int NPW, bool Q41>
 __device__ __forceinline__ void subtree(const GuTile &t, const GuStage &g, uint32_t w_off, int wave, int lane,
                                         uint4 (&wn)[2], float (&res)[16]) {
@@ -751,8 +751,8 @@ void launch_linear_mfma_t(const LinearArgsOf<Q41> &a, hipStream_t s) {
     constexpr unsigned T = 64 * W;
     const unsigned grid = static_cast<unsigned>((a.row_tiles + 7) / 8 * 8) * static_cast<unsigned>(a.col_tiles);
     // Only 64-block rows take the 8-wave form: for the other folds the
-    // compiler's register allocator (with the iterative-ILP scheduler this
-    // file is built with) fails on it.
+    // compiler's register allocator fails on it (with the iterative-ILP
+    // scheduler that moe_mfma.hip is built with).
     if (a.nb == kGuMaxBlocks) k_linear_mfma<kFoldGrouped, Canon, W, Q41><<<grid, T, 0, s>>>(a);
     else if (a.nb > kGuMaxBlocks && a.nb <= kGu96MaxBlocks) k_linear_mfma<kFoldGrouped96, Canon, 4, Q41><<<grid, 256, 0, s>>>(a);
     else if (a.nb < kGuMaxBlocks) k_linear_mfma<kFoldStaged, Canon, 4, Q41><<<grid, 256, 0, s>>>(a);

@@ -254,8 +254,8 @@ __device__ __forceinline__ void tile_dispatch(const TileArgs &t, int nsub, float
 // 3.54 -> 2.98 ms with Q4_1, against kFoldMulti; the fp16-operand form with a
 // third block pair, two waves per SIMD at 63 KB of LDS, measured 3 % slower)
 // or kFoldMulti (H > 3072); one instantiation per shape keeps only that
-// path's registers.  The linear kernel below also takes kFoldStaged (< 64
-// blocks) and kFoldGrouped (64).
+// path's registers.  The linear kernel (moe_leaf.hpp) also takes kFoldStaged
+// (< 64 blocks) and kFoldGrouped (64).
 template<int Fold, bool Dbg>
 __global__ __launch_bounds__(128, 2) void k_gate_up_mfma(FfnArgs a) {
     // Pending tree levels 3-4 per wave; after the tree, the waves' results.
